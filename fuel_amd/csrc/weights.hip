@@ -5,8 +5,10 @@
 // and with from_float_imatrix for Q4_K and Q6_K (quantize_imatrix:
 // k_quants.rs:1530-1593 with make_qkx3_quants utils.rs:358-469 and
 // make_qp_quants utils.rs:472-563; k_quants.rs:2077-2145).
-// One thread per superblock runs the reference's sequential float search in the
-// same operation order (built with -ffp-contract=off; '/' is IEEE-correct).
+// One thread per scale group (Q4_K sub-block of 32, Q6_K group of 16; per
+// superblock for the Q4_K imatrix search) runs the reference's sequential float
+// search in the same operation order (built with -ffp-contract=off; '/' is
+// IEEE-correct), and the lanes of a superblock share the scales by shuffles.
 //
 // Also the synthetic-input generator: Philox-4x32-10 words
 // (fuel-cpu-kernels/src/philox.rs:47-135) and a Box-Muller normal transform.
@@ -26,6 +28,26 @@ __device__ __forceinline__ int total_key(float f) {
     return b ^ (int)(((unsigned)(b >> 31)) >> 1);
 }
 
+// clamp(nearest_int(v), 0, 15) as a float: rounding and clamping commute, NaN
+// gives 0 as nearest_int does, and truncating w + 0.49999997 rounds half away
+// from zero for every float in [0, 15].
+__device__ __forceinline__ float round_0_15(float v) {
+    return __builtin_truncf(fminf(fmaxf(v, 0.0f), 15.0f) + 0.49999997f);
+}
+// clamp(nearest_int(v), -32, 31): the same rounding; the integer conversion
+// saturates and takes NaN to 0, as nearest_int does.
+__device__ __forceinline__ int round_m32_31(float v) {
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(v + __builtin_copysignf(0.49999997f, v)));
+    return clampi(i, -32, 31);
+}
+// Whether a quotient num * rcp(den) may round to another integer than the IEEE
+// quotient.  The two are within 4 ulp (1.5e-5 below 64; larger ones are
+// clamped), so only if it lies that close to a half integer; or it is not
+// finite (rcp of a denormal, 0 / 0).  den must be below 2^126, where rcp would
+// be flushed to zero.
+__device__ __forceinline__ bool near_half(float t) { return !(fabsf(t - floorf(t) - 0.5f) > 2e-5f); }
+
 // make_qkx1_quants(nmax = 15, ntry = 5, x[32]) -> (scale, -min)
 __device__ void make_qkx1_quants_15_5(const float (&x)[32], float& out_scale, float& out_min) {
     float mn = x[0], mx = x[0];
@@ -44,26 +66,25 @@ __device__ void make_qkx1_quants_15_5(const float (&x)[32], float& out_scale, fl
     float min = fminf(mn, 0.0f);
     float iscale = 15.0f / (mx - min);
     float scale = 1.0f / iscale;
-    uint32_t l[4] = {0u, 0u, 0u, 0u};  // 32 nibbles
+    float l[32];  // the codes (small integers, exact; sums of their squares too)
+#pragma unroll
+    for (int i = 0; i < 32; i++) l[i] = 0.0f;
     for (int t = 0; t < 5; t++) {
-        float sumlx = 0.0f;
-        int suml2 = 0;
-        bool changed = false;
+        float sumlx = 0.0f, suml2 = 0.0f;
+        uint32_t changed = 0u;
 #pragma unroll
         for (int i = 0; i < 32; i++) {
-            const int li = clampi(nearest_int(iscale * (x[i] - min)), 0, 15);
-            const uint32_t old = (l[i >> 3] >> (4 * (i & 7))) & 0xfu;
-            if ((uint32_t)li != old) {
-                l[i >> 3] = (l[i >> 3] & ~(0xfu << (4 * (i & 7)))) | ((uint32_t)li << (4 * (i & 7)));
-                changed = true;
-            }
-            sumlx += (x[i] - min) * (float)li;
-            suml2 += li * li;
+            const float xm = x[i] - min;
+            const float li = round_0_15(iscale * xm);
+            changed |= __builtin_bit_cast(uint32_t, li) ^ __builtin_bit_cast(uint32_t, l[i]);
+            l[i] = li;
+            sumlx += xm * li;
+            suml2 = fmaf(li, li, suml2);
         }
-        scale = sumlx / (float)suml2;
+        scale = sumlx / suml2;
         float sum = -0.0f;
 #pragma unroll
-        for (int i = 0; i < 32; i++) sum += x[i] - scale * (float)((l[i >> 3] >> (4 * (i & 7))) & 0xfu);
+        for (int i = 0; i < 32; i++) sum += x[i] - scale * l[i];
         min = sum / 32.0f;
         if (min > 0.0f) min = 0.0f;
         iscale = 1.0f / scale;
@@ -115,7 +136,7 @@ __device__ float make_qx_quants_16(const float (&x)[16], int (&ls)[16], const fl
     float sumlx = 0.0f, suml2 = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        const int l = clampi(nearest_int(iscale * x[i]), -32, 31);
+        const int l = round_m32_31(iscale * x[i]);
         ls[i] = l + 32;
         const float w = qw ? qw[i] : x[i] * x[i];
         const float lf = (float)l;
@@ -130,7 +151,7 @@ __device__ float make_qx_quants_16(const float (&x)[16], int (&ls)[16], const fl
         bool changed = false;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int l = clampi(nearest_int(is2 * x[i]), -32, 31);
+            const int l = round_m32_31(is2 * x[i]);
             if (l + 32 != ls[i]) changed = true;
             const float w = qw ? qw[i] : x[i] * x[i];
             const float lf = (float)l;
@@ -139,7 +160,7 @@ __device__ float make_qx_quants_16(const float (&x)[16], int (&ls)[16], const fl
         }
         if (!changed || sl2 == 0.0f || slx * slx <= best * sl2) break;
 #pragma unroll
-        for (int i = 0; i < 16; i++) ls[i] = 32 + clampi(nearest_int(is2 * x[i]), -32, 31);
+        for (int i = 0; i < 16; i++) ls[i] = 32 + round_m32_31(is2 * x[i]);
         sumlx = slx;
         suml2 = sl2;
         scale = sumlx / suml2;
@@ -154,7 +175,8 @@ __device__ float make_qx_quants_16(const float (&x)[16], int (&ls)[16], const fl
             float slx = sumlx - w * x[i] * (float)l;
             if (slx > 0.0f) {
                 float sl2 = suml2 - w * (float)l * (float)l;
-                const int new_l = clampi(nearest_int(x[i] * sl2 / slx), -32, 31);
+                const float num = x[i] * sl2, q = num * __builtin_amdgcn_rcpf(slx);
+                const int new_l = round_m32_31(near_half(q) || slx > 1e37f ? num / slx : q);
                 if (new_l != l) {
                     slx += w * x[i] * (float)new_l;
                     sl2 += w * (float)new_l * (float)new_l;
@@ -354,42 +376,89 @@ __device__ float make_qp_quants_8(const float (&x)[8], int (&l)[8], const float 
 
 }  // namespace
 
-// One thread per 256-element superblock.
-__global__ __launch_bounds__(64) void quantize_q4k_weights_kernel(const float* __restrict__ x, size_t nblocks,
-                                                                  uint8_t* __restrict__ out) {
-    const size_t ib = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (ib >= nblocks) return;
-    const float* xb = x + ib * QK_K;
-    float scales[8], mins[8];
-    for (int j = 0; j < 8; j++) {
-        float v[32];
-        load32(xb + 32 * j, v);
-        make_qkx1_quants_15_5(v, scales[j], mins[j]);
+// Lane 8 b + j of a wavefront: sub-block j of the wavefront's superblock b, its
+// 32 values in registers.  The search is VALU bound: 13 operations a value and
+// round.  One thread per superblock, with every value read twice, took 310 us
+// for 11008 x 4096 (two wavefronts a SIMD); this takes 120 us.
+__global__ __launch_bounds__(256) void quantize_q4k_weights_kernel(const float* __restrict__ x, size_t nblocks,
+                                                                   uint8_t* __restrict__ out) {
+    const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x, ib = g >> 3;
+    if (ib >= nblocks) return;  // (whole groups of eight lanes)
+    const int j = threadIdx.x & 7;
+    float v[32];
+    load32(x + 32 * g, v);
+    float scale, mn;
+    make_qkx1_quants_15_5(v, scale, mn);
+    float max_scale = fmaxf(scale, 0.0f), max_min = fmaxf(mn, 0.0f);
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        max_scale = fmaxf(max_scale, __shfl_xor(max_scale, o));
+        max_min = fmaxf(max_min, __shfl_xor(max_min, o));
     }
-    float max_scale = 0.0f, max_min = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) max_scale = fmaxf(scales[j], max_scale);
-#pragma unroll
-    for (int j = 0; j < 8; j++) max_min = fmaxf(mins[j], max_min);
     const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
     const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
+    const int a = nearest_int(inv_scale * scale), c = nearest_int(inv_min * mn);
+    const int both = (int)(uint8_t)(a < 63 ? a : 63) | ((int)(uint8_t)(c < 63 ? c : 63) << 8);
     uint8_t sc[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int a = nearest_int(inv_scale * scales[j]);
-        const int c = nearest_int(inv_min * mins[j]);
-        const uint8_t ls = (uint8_t)(a < 63 ? a : 63);
-        const uint8_t lm = (uint8_t)(c < 63 ? c : 63);
-        if (j < 4) {
-            sc[j] = ls;
-            sc[j + 4] = lm;
+    for (int i = 0; i < 8; i++) {
+        const int t = __shfl(both, i, 8);
+        const uint8_t ls = (uint8_t)t, lm = (uint8_t)(t >> 8);
+        if (i < 4) {
+            sc[i] = ls;
+            sc[i + 4] = lm;
         } else {
-            sc[j + 4] = (uint8_t)((ls & 0xF) | ((lm & 0xF) << 4));
-            sc[j - 4] |= (uint8_t)((ls >> 4) << 6);
-            sc[j] |= (uint8_t)((lm >> 4) << 6);
+            sc[i + 4] = (uint8_t)((ls & 0xF) | ((lm & 0xF) << 4));
+            sc[i - 4] |= (uint8_t)((ls >> 4) << 6);
+            sc[i] |= (uint8_t)((lm >> 4) << 6);
         }
     }
-    q4k_store(xb, sc, f32_to_f16_rne(max_scale / 63.0f), f32_to_f16_rne(max_min / 63.0f), out + ib * Q4K_BYTES);
+    const uint16_t dh = f32_to_f16_rne(max_scale / 63.0f), mh = f32_to_f16_rne(max_min / 63.0f);
+    int s = 0, m = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        int si, mi;
+        scale_min_k4(i, sc, si, mi);
+        s = i == j ? si : s;
+        m = i == j ? mi : m;
+    }
+    // the codes as bytes, the odd sub-blocks' in the high nibbles
+    const float d = f16_to_f32(dh) * (float)s, dm = f16_to_f32(mh) * (float)m;
+    uint32_t words[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (d != 0.0f) {  // (else L stays 0)
+        const float rd = __builtin_amdgcn_rcpf(d);
+        const int sh = 4 * (j & 1);
+        bool near = false;
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            const float q = (v[i] + dm) * rd;
+            near |= near_half(q);
+            words[i >> 2] |= (uint32_t)round_0_15(q) << (8 * (i & 3));
+        }
+        if (near) {
+#pragma unroll
+            for (int w = 0; w < 8; w++) {
+                words[w] = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) words[w] |= (uint32_t)round_0_15((v[4 * w + i] + dm) / d) << (8 * i);
+            }
+        }
+#pragma unroll
+        for (int w = 0; w < 8; w++) words[w] <<= sh;
+    }
+#pragma unroll
+    for (int w = 0; w < 8; w++) words[w] |= (uint32_t)__shfl_xor((int)words[w], 1);
+    uint8_t* ob = out + ib * Q4K_BYTES;
+    if (j == 0) {
+        uint32_t h[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            h[i] = (uint32_t)sc[4 * i] | ((uint32_t)sc[4 * i + 1] << 8) | ((uint32_t)sc[4 * i + 2] << 16) |
+                   ((uint32_t)sc[4 * i + 3] << 24);
+        *reinterpret_cast<uint4*>(ob) = uint4{(uint32_t)dh | ((uint32_t)mh << 16), h[0], h[1], h[2]};
+    }
+    *reinterpret_cast<uint4*>(ob + 16 + 16 * j) =
+        j & 1 ? uint4{words[4], words[5], words[6], words[7]} : uint4{words[0], words[1], words[2], words[3]};
 }
 
 // from_float_imatrix for Q4_K, one thread per superblock: sub-block j's
@@ -441,87 +510,77 @@ __global__ __launch_bounds__(64) void quantize_q4k_imatrix_kernel(const float* _
     q4k_store(xb, sc, f32_to_f16_rne(d_block), f32_to_f16_rne(m_block), out + ib * Q4K_BYTES);
 }
 
-// One thread per superblock; the 256 codes L live in LDS (256 B per thread).
-// With imatrix set (from_float_imatrix), superblock ib's groups are weighted by
-// imatrix[(ib % bpr) * 256 ...] instead of x * x.
-__global__ __launch_bounds__(64) void quantize_q6k_weights_kernel(const float* __restrict__ x, size_t nblocks,
-                                                                  uint8_t* __restrict__ out,
-                                                                  const float* __restrict__ imatrix, size_t bpr) {
-    __shared__ int8_t Ls[64][QK_K];
-    const size_t ib = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (ib >= nblocks) return;
-    int8_t* L = Ls[threadIdx.x];
-    const float* xb = x + ib * QK_K;
-    float scales[16];
-    float max_scale = 0.0f, max_abs_scale = 0.0f;
-    for (int g = 0; g < 16; g++) {
-        float v[16];
+// Lane 16 b + g of a wavefront: 16-element group g of the wavefront's
+// superblock b; the superblock's 256 codes meet in LDS, where its 16 lanes turn
+// them into the block's bytes.  With imatrix set (from_float_imatrix),
+// superblock ib's groups are weighted by imatrix[(ib % bpr) * 256 ...] instead
+// of x * x.  VALU bound; one thread per superblock took 361 us for 4096 x 4096,
+// this takes 94 us.
+__global__ __launch_bounds__(256) void quantize_q6k_weights_kernel(const float* __restrict__ x, size_t nblocks,
+                                                                   uint8_t* __restrict__ out,
+                                                                   const float* __restrict__ imatrix, size_t bpr) {
+    __shared__ __align__(16) uint8_t Ls[16][QK_K + 16];
+    const size_t gi = (size_t)blockIdx.x * 256 + threadIdx.x, ib = gi >> 4;
+    const bool live = ib < nblocks;  // (whole groups of 16 lanes)
+    const int g = threadIdx.x & 15;
+    uint8_t* L = Ls[threadIdx.x >> 4];
+    float v[16];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float4 t = reinterpret_cast<const float4*>(xb + 16 * g)[i];
-            v[4 * i] = t.x;
-            v[4 * i + 1] = t.y;
-            v[4 * i + 2] = t.z;
-            v[4 * i + 3] = t.w;
-        }
-        int ls[16];
-        const float s = make_qx_quants_16(v, ls, imatrix ? imatrix + (ib % bpr) * QK_K + 16 * g : nullptr);
+    for (int i = 0; i < 4; i++) {
+        const float4 t = live ? reinterpret_cast<const float4*>(x + 16 * gi)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[4 * i] = t.x;
+        v[4 * i + 1] = t.y;
+        v[4 * i + 2] = t.z;
+        v[4 * i + 3] = t.w;
+    }
+    int ls[16];
+    const float scale = make_qx_quants_16(v, ls, imatrix ? imatrix + (ib % bpr) * QK_K + 16 * g : nullptr);
+    float max_scale = 0.0f, max_abs_scale = 0.0f;  // the first group of the largest |scale|
 #pragma unroll
-        for (int i = 0; i < 16; i++) L[16 * g + i] = (int8_t)ls[i];
-        scales[g] = s;
-        const float as = fabsf(s);
-        if (as > max_abs_scale) {
-            max_abs_scale = as;
-            max_scale = s;
-        }
+    for (int i = 0; i < 16; i++) {
+        const float t = __shfl(scale, i, 16), at = fabsf(t);
+        max_scale = at > max_abs_scale ? t : max_scale;
+        max_abs_scale = at > max_abs_scale ? at : max_abs_scale;
     }
     const float iscale = -128.0f / max_scale;
     const uint16_t dh = f32_to_f16_rne(1.0f / iscale);
-    const float df = f16_to_f32(dh);
-    int8_t sc[16];
+    const int si = nearest_int(iscale * scale);
+    const int8_t sc = (int8_t)(si < 127 ? si : 127);
+    const float d = f16_to_f32(dh) * (float)sc;
+    if (d != 0.0f) {  // (else the search's codes stay)
+        const float rd = __builtin_amdgcn_rcpf(d);
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const int v = nearest_int(iscale * scales[j]);
-        sc[j] = (int8_t)(v < 127 ? v : 127);
-    }
-    for (int j = 0; j < 16; j++) {
-        const float d = df * (float)sc[j];
-        if (d == 0.0f) continue;
-        float v[16];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float4 t = reinterpret_cast<const float4*>(xb + 16 * j)[i];
-            v[4 * i] = t.x;
-            v[4 * i + 1] = t.y;
-            v[4 * i + 2] = t.z;
-            v[4 * i + 3] = t.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; i++) L[16 * j + i] = (int8_t)(clampi(nearest_int(v[i] / d), -32, 31) + 32);
-    }
-    uint8_t* ob = out + ib * Q6K_BYTES;  // only 2-byte aligned: 16-bit stores
-    for (int h = 0; h < 2; h++) {
-        const int8_t* Lh = L + 128 * h;
-        for (int l = 0; l < 32; l += 2) {
-            uint8_t qlA[2], qlB[2], qhv[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int i = l + t;
-                const uint8_t q1 = (uint8_t)(Lh[i] & 0xF), q2 = (uint8_t)(Lh[i + 32] & 0xF);
-                const uint8_t q3 = (uint8_t)(Lh[i + 64] & 0xF), q4 = (uint8_t)(Lh[i + 96] & 0xF);
-                qlA[t] = (uint8_t)(q1 | (q3 << 4));
-                qlB[t] = (uint8_t)(q2 | (q4 << 4));
-                qhv[t] = (uint8_t)((Lh[i] >> 4) | ((Lh[i + 32] >> 4) << 2) | ((Lh[i + 64] >> 4) << 4) |
-                                   ((Lh[i + 96] >> 4) << 6));
-            }
-            *reinterpret_cast<uint16_t*>(ob + 64 * h + l) = (uint16_t)(qlA[0] | (qlA[1] << 8));
-            *reinterpret_cast<uint16_t*>(ob + 64 * h + 32 + l) = (uint16_t)(qlB[0] | (qlB[1] << 8));
-            *reinterpret_cast<uint16_t*>(ob + 128 + 32 * h + l) = (uint16_t)(qhv[0] | (qhv[1] << 8));
+        for (int i = 0; i < 16; i++) {
+            const float q = v[i] * rd;
+            ls[i] = round_m32_31(near_half(q) ? v[i] / d : q) + 32;
         }
     }
-    for (int j = 0; j < 16; j += 2)
-        *reinterpret_cast<uint16_t*>(ob + 192 + j) = (uint16_t)((uint8_t)sc[j] | ((uint8_t)sc[j + 1] << 8));
-    *reinterpret_cast<uint16_t*>(ob + 208) = dh;
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        w[i] = (uint32_t)(ls[4 * i] & 0xff) | ((uint32_t)(ls[4 * i + 1] & 0xff) << 8) |
+               ((uint32_t)(ls[4 * i + 2] & 0xff) << 16) | ((uint32_t)(ls[4 * i + 3] & 0xff) << 24);
+    *reinterpret_cast<uint4*>(L + 16 * g) = uint4{w[0], w[1], w[2], w[3]};
+    __syncthreads();
+    if (!live) return;
+    // lane g: bytes 8 (g & 7) .. + 7 of half g >> 3's 64 ql bytes and bytes
+    // 4 (g & 7) .. + 3 of its 32 qh bytes (blocks are only 2-byte aligned)
+    const int h = g >> 3, l = 4 * (g & 7);
+    uint32_t c[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) c[i] = *reinterpret_cast<const uint32_t*>(L + 128 * h + 32 * i + l);
+    uint8_t* ob = out + ib * Q6K_BYTES;
+    auto put4 = [](uint8_t* p, uint32_t b) __attribute__((always_inline)) {
+        reinterpret_cast<uint16_t*>(p)[0] = (uint16_t)b;
+        reinterpret_cast<uint16_t*>(p)[1] = (uint16_t)(b >> 16);
+    };
+    put4(ob + 64 * h + l, (c[0] & 0x0f0f0f0fu) | ((c[2] & 0x0f0f0f0fu) << 4));
+    put4(ob + 64 * h + 32 + l, (c[1] & 0x0f0f0f0fu) | ((c[3] & 0x0f0f0f0fu) << 4));
+    // (codes are 0..63; the reference shifts whole signed bytes)
+    put4(ob + 128 + 32 * h + l, ((c[0] >> 4) & 0x0f0f0f0fu) | (((c[1] >> 4) & 0x0f0f0f0fu) << 2) |
+                                    (((c[2] >> 4) & 0x0f0f0f0fu) << 4) | (((c[3] >> 4) & 0x03030303u) << 6));
+    ob[192 + g] = (uint8_t)sc;
+    if (g == 0) *reinterpret_cast<uint16_t*>(ob + 208) = dh;
 }
 
 // Eight 32-element blocks per wavefront (the activation quantizer's arithmetic).
@@ -543,11 +602,11 @@ hipError_t launch_quantize_weights(int dtype, const float* x, size_t nblocks, ui
     if (nblocks == 0) return hipSuccess;
     switch (dtype) {
         case GGML_Q4K:
-            hipLaunchKernelGGL(quantize_q4k_weights_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(64), 0, s, x,
+            hipLaunchKernelGGL(quantize_q4k_weights_kernel, dim3((unsigned)((nblocks + 31) / 32)), dim3(256), 0, s, x,
                                nblocks, out);
             break;
         case GGML_Q6K:
-            hipLaunchKernelGGL(quantize_q6k_weights_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(64), 0, s, x,
+            hipLaunchKernelGGL(quantize_q6k_weights_kernel, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0, s, x,
                                nblocks, out, nullptr, (size_t)1);
             break;
         case GGML_Q8_0:
@@ -563,15 +622,14 @@ hipError_t launch_quantize_weights_imatrix(int dtype, const float* x, size_t nbl
                                            size_t blocks_per_row, uint8_t* out, hipStream_t s) {
     if (nblocks == 0) return hipSuccess;
     if (blocks_per_row == 0 || !imatrix) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((nblocks + 63) / 64));
     switch (dtype) {
         case GGML_Q4K:
-            hipLaunchKernelGGL(quantize_q4k_imatrix_kernel, grid, dim3(64), 0, s, x, nblocks, out, imatrix,
+            hipLaunchKernelGGL(quantize_q4k_imatrix_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(64), 0, s, x, nblocks, out, imatrix,
                                blocks_per_row);
             break;
         case GGML_Q6K:
-            hipLaunchKernelGGL(quantize_q6k_weights_kernel, grid, dim3(64), 0, s, x, nblocks, out, imatrix,
-                               blocks_per_row);
+            hipLaunchKernelGGL(quantize_q6k_weights_kernel, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0, s, x,
+                               nblocks, out, imatrix, blocks_per_row);
             break;
         default: return hipErrorInvalidValue;
     }

@@ -344,6 +344,45 @@ def test_device_quantize_bit_exact(dev, dt):
     assert got.tobytes() == want.tobytes(), f"first differing blocks {np.unique(bad[0])[:8]}"
 
 
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+@pytest.mark.parametrize("blocks", [1, 7, 9, 33])
+def test_device_quantize_few_blocks(dev, dt, blocks):
+    """Block counts that end inside a wavefront and a workgroup, and rows whose
+    quotients meet the rounding edge cases: half-integer ties, tiny and huge
+    magnitudes, rows of one repeated value, mostly-zero rows.  Byte for byte,
+    and the blocks back to f32 / f16 bit for bit."""
+    say("device from_float, few blocks", dt, blocks)
+    rng = np.random.default_rng(blocks)
+    rows = []
+    for i in range(blocks):
+        x = rng.standard_normal(256).astype(np.float32)
+        kind = i % 7
+        if kind == 1:
+            x = (rng.integers(-31, 32, 256) * np.float32(0.5)).astype(np.float32)  # halves of the grid
+        elif kind == 2:
+            x *= np.float32(1e-30)
+        elif kind == 3:
+            x *= np.float32(1e9)
+        elif kind == 4:
+            x[:] = np.float32(-0.75)
+        elif kind == 5:
+            x[rng.random(256) < 0.95] = 0
+        elif kind == 6:
+            x = np.abs(x) * np.float32(1e-6)
+        rows.append(x)
+    w = np.concatenate(rows)[None]
+    want = O.quantize(dt, w)
+    q = dev.qzeros(w.size, dt)
+    q.quantize(dev.from_numpy(w))
+    got = np.frombuffer(q.data(), O.BLOCK_DTYPE[dt]).reshape(want.shape)
+    bad = np.nonzero(got.view(np.uint8).reshape(got.size, -1) != want.view(np.uint8).reshape(want.size, -1))
+    assert got.tobytes() == want.tobytes(), f"first differing blocks {np.unique(bad[0])[:8]}"
+    values = O.dequantize(dt, want).reshape(-1)
+    assert np.array_equal(q.dequantize(w.size).numpy().view(np.uint32), values.view(np.uint32))
+    with np.errstate(over="ignore"):
+        assert np.array_equal(q.dequantize_f16(w.size).numpy(), values.astype(np.float16).view(np.uint16))
+
+
 def test_device_quantize_known_answers(dev):
     """The hand-derived known-answer blocks of weight_kat.py (grid-exact
     sub-blocks, clamps, ties, saturation, zero blocks) through the device
