@@ -179,7 +179,15 @@ struct MmqGroup {
     const uint8_t* w2;
     int n_split;
 };
-int mmq_group_rows(int rows_per_expert);  // tile height for an average rows-per-expert
+// Tile height for an average rows-per-expert.  wide: every operand allows the
+// grouped wide-tile kernel (Q4_K blocks at 16-byte aligned bases, a W | W2
+// split that is a multiple of its 128 columns): from two rows per expert on
+// average (128 experts, top-8, 2048 / 768, the whole layer: 32 tokens 99.8 ->
+// 99.1 us, 192 126 -> 117, 256 141 -> 123, 512 181 -> 147, 1024 293 -> 224
+// against the 16- and 32-row tiles; below two the 16-row tiles, 20 tokens 85.8
+// against 88.3).
+constexpr int MMQ_GROUP_WIDE_ROWS = 64, MMQ_GROUP_WIDE_MIN = 2;
+int mmq_group_rows(int dtype, int rows_per_expert, bool wide);
 hipError_t launch_mmq_grouped(int dtype, const uint8_t* w, ActView act, float* y, int bm, int max_tiles, int N, int K,
                               int ldy, const MmqGroup& g, hipStream_t s);
 // Per-(m, n, block) integer sums, the bit-exact stage of the dot products.

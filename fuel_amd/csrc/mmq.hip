@@ -917,6 +917,175 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
         }
 }
 
+// ---- Q4_K, grouped (MoE) wide tiles ----
+// The wide-tile computation for the expert-sorted rows: workgroup (x, c) takes
+// tile x of the tile table (up to 64 rows of one expert) and 128 columns of
+// that expert's weights (128-column tiles lie on one side of the W | W2 split).
+// Activation rows are gathered by the DMA's per-lane offsets.  A tile is as
+// tall as an expert's rows usually reach, so an expert's blocks are read and
+// unpacked once, and the wavefronts work only the 16-row parts that hold rows
+// (RL of them, one code path each): the kernel is bound by its VALU work,
+// mostly the unpacking, which does not depend on the rows.  (Q4K 128 experts,
+// 4096 routed rows, 2048 -> 2 x 768 -> 2048: gate|up 111 -> 75 us, down 61 ->
+// 49 us against 32-row tiles of the register-staged kernel, where experts of
+// 33 or more rows take two tiles and each product three MFMAs.)
+constexpr int GRP_RT = 4, GRP_NW = 8;
+
+__global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint8_t* __restrict__ W, ActView act,
+                                                                      float* __restrict__ y, int N, int K, int ldy,
+                                                                      MmqGroup g) {
+    constexpr int RT = GRP_RT, NW = GRP_NW;
+    using T = WideTile<RT, 1, NW>;
+    constexpr int BM = T::BM, BN = T::BN;
+    static_assert(T::CA == 2 * NW && T::CS == 2 && T::CD == 1 && T::CW == 18, "the DMA deal below");
+    __shared__ __align__(16) uint8_t sB0[T::LBUF], sB1[T::LBUF];
+
+    if ((int)blockIdx.x >= *g.ntiles) return;  // uniform: the tile table is shorter than the grid bound
+    const int e = __builtin_amdgcn_readfirstlane(g.tile_expert[blockIdx.x]);
+    const int m0 = __builtin_amdgcn_readfirstlane(g.tile_row0[blockIdx.x]);
+    const int rows = min(BM, __builtin_amdgcn_readfirstlane(g.expert_offsets[e + 1]) - m0);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KB = K / QK_K;
+    const uint32_t row_bytes = (uint32_t)KB * Q4K_BYTES;
+    const int l16 = lane & 15, kb = lane >> 4;
+    const int n0 = blockIdx.y * BN;
+    const bool second = g.w2 && n0 >= g.n_split;  // the tile's columns lie on one side of the split
+    const uint8_t* We = (second ? g.w2 : W) + (size_t)e * g.expert_bytes;
+    const int nbase = second ? n0 - g.n_split : n0;
+    const int nlast = (second ? N - g.n_split : g.w2 ? g.n_split : N) - 1;
+
+    // DMA sources (superblock 0).  Activation instruction i = 8 j + wave covers
+    // rows 4 i .. 4 i + 3; rows past the expert's read row m0's (valid bytes,
+    // outputs never stored).  Weight chunks: 18 instructions, wavefronts 0 and
+    // 1 take three; the 16-element sums go to wavefronts 2 and 3, the scales to
+    // wavefront 4.
+    auto row_of = [&](int r) { const int m = m0 + (r < rows ? r : 0); return g.x_row ? g.x_row[m] : m; };
+    uint32_t asrc[2], wsrc[3];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int r = 4 * (j * NW + wave) + (lane >> 4);
+        asrc[j] = (uint32_t)row_of(r) * (uint32_t)K + 16u * (uint32_t)((lane & 15) ^ (r & 15));
+    }
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int q = 64 * (j * NW + wave) + lane;  // (j = 2: wavefronts 0 and 1 only)
+        const int n = min(nbase + q / 9, nlast);
+        wsrc[j] = (uint32_t)n * row_bytes + 16u * (uint32_t)(q % 9);
+    }
+    uint32_t xsrc = 0;  // sums or scales
+    if (wave == 2 || wave == 3) xsrc = 32u * (uint32_t)row_of(32 * (wave - 2) + (lane >> 1)) * (uint32_t)KB + 16u * (uint32_t)(lane & 1);
+    if (wave == 4) xsrc = 4u * (uint32_t)row_of(lane) * (uint32_t)KB;
+    const uint8_t* qbase = reinterpret_cast<const uint8_t*>(act.qs);
+    const uint8_t* sbase = reinterpret_cast<const uint8_t*>(act.bsh);
+    const uint8_t* dbase = reinterpret_cast<const uint8_t*>(act.d);
+
+    const uint32_t sel0 = (uint32_t)(2 * (kb >> 1)) * 0x00010001u | 0x0c000c00u;
+    const uint32_t sel1 = sel0 + 0x00010001u;
+    const uint32_t msel = (uint32_t)(2 * (kb & 1)) * 0x01010101u + 0x01010000u;
+    const uint32_t slot0 = lds_addr(sB0), slot1 = lds_addr(sB1);
+
+    auto run = [&](auto rl) __attribute__((always_inline)) {
+        constexpr int RL = decltype(rl)::value;
+        auto issue = [&](int b, uint32_t buf) __attribute__((always_inline)) {
+            const uint32_t ub = (uint32_t)b;
+            dma16_asm(qbase, asrc[0] + ub * QK_K, buf + (uint32_t)(1024 * wave));
+            if (RL > 2) dma16_asm(qbase, asrc[1] + ub * QK_K, buf + (uint32_t)(1024 * (NW + wave)));
+            dma16_asm(We, wsrc[0] + ub * Q4K_BYTES, buf + (uint32_t)(T::OW + 1024 * wave));
+            dma16_asm(We, wsrc[1] + ub * Q4K_BYTES, buf + (uint32_t)(T::OW + 1024 * (NW + wave)));
+            if (wave < 2) dma16_asm(We, wsrc[2] + ub * Q4K_BYTES, buf + (uint32_t)(T::OW + 1024 * (2 * NW + wave)));
+            else if (wave < 4) dma16_asm(sbase, xsrc + ub * 32u, buf + (uint32_t)(T::OS + 1024 * (wave - 2)));
+            else if (wave == 4) dma4_asm(dbase, xsrc + ub * 4u, buf + (uint32_t)T::OD);
+        };
+        float facc[RL][4];
+#pragma unroll
+        for (int r = 0; r < RL; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) facc[r][i] = 0.0f;
+        issue(0, slot0);
+        auto iter = [&](auto kr, int b) __attribute__((always_inline)) {
+            constexpr int KR = decltype(kr)::value;
+            const uint8_t* A = KR == 0 ? sB0 : sB1;
+            const uint8_t* S = A + T::OS;
+            const float* D = reinterpret_cast<const float*>(A + T::OD);
+            // superblock b landed in every wavefront; the other slot's readers have left iteration b - 1
+            __builtin_amdgcn_s_waitcnt(FRQ_VMCNT(0));
+            compiler_fence();
+            __builtin_amdgcn_s_barrier();
+            compiler_fence();
+            if (b + 1 < KB) issue(b + 1, KR == 0 ? slot1 : slot0);
+            const uint8_t* col = A + T::OW + (16 * wave + l16) * Q4K_BYTES;
+            const uint4 hd = *reinterpret_cast<const uint4*>(col);
+            const uint32_t sc0 = hd.y & 0x3f3f3f3fu;
+            const uint32_t sc1 = (hd.w & 0x0f0f0f0fu) | (((hd.y >> 6) & 0x03030303u) << 4);
+            const uint32_t mn = kb < 2 ? hd.z & 0x3f3f3f3fu
+                                       : ((hd.w >> 4) & 0x0f0f0f0fu) | (((hd.z >> 6) & 0x03030303u) << 4);
+            const float d = f16_to_f32(hd.x & 0xffffu), dmin = f16_to_f32(hd.x >> 16);
+            const uint32_t aw[2] = {(sc0 >> 3) & 0x07070707u, (sc1 >> 3) & 0x07070707u};
+            const uint32_t bw[2] = {sc0 & 0x07070707u, sc1 & 0x07070707u};
+            v4i acc[RL][2];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int j = 8 * (t & 1) + 4 * (kb >> 1) + 2 * (t >> 1) + (kb & 1);  // activation chunk
+                v4i afr[RL];
+#pragma unroll
+                for (int r = 0; r < RL; r++)
+                    afr[r] = *reinterpret_cast<const v4i*>(A + (16 * r + l16) * QK_K + 16 * (j ^ l16));
+                const uint4 rw = *reinterpret_cast<const uint4*>(col + 16 + 64 * (t & 1) + 16 * kb);
+                const uint32_t sh = t >= 2 ? 4u : 0u;
+                const uint32_t qd[4] = {(rw.x >> sh) & 0x0f0f0f0fu, (rw.y >> sh) & 0x0f0f0f0fu,
+                                        (rw.z >> sh) & 0x0f0f0f0fu, (rw.w >> sh) & 0x0f0f0f0fu};
+                const uint32_t sel = t >= 2 ? sel1 : sel0;
+                const uint32_t pa = byte_pair(aw[t & 1], sel), pb = byte_pair(bw[t & 1], sel);
+                const v4i ba = v4i{bytes_times_p(qd[0], pa), bytes_times_p(qd[1], pa), bytes_times_p(qd[2], pa),
+                                   bytes_times_p(qd[3], pa)};
+                const v4i bb = v4i{bytes_times_p(qd[0], pb), bytes_times_p(qd[1], pb), bytes_times_p(qd[2], pb),
+                                   bytes_times_p(qd[3], pb)};
+                const v4i zero = v4i{0, 0, 0, 0};
+#pragma unroll
+                for (int r = 0; r < RL; r++) {
+                    acc[r][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(afr[r], ba, t == 0 ? zero : acc[r][0], 0, 0, 0);
+                    acc[r][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(afr[r], bb, t == 0 ? zero : acc[r][1], 0, 0, 0);
+                }
+            }
+            // msum on f16 MFMA, then the f32 step (the wide-tile kernel's)
+            const uint32_t mm = __builtin_amdgcn_perm(0u, mn, msel);  // bytes m_lo, m_lo, m_hi, m_hi
+            const wh4 mb = wh4{(_Float16)(mm & 0xffu), (_Float16)((mm >> 8) & 0xffu), (_Float16)((mm >> 16) & 0xffu),
+                               (_Float16)(mm >> 24)};
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                const wh4 sa = *reinterpret_cast<const wh4*>(S + (16 * r + l16) * 32 + 8 * kb);  // b_{4kb..4kb+3}
+                const float4 dx = *reinterpret_cast<const float4*>(D + 16 * r + 4 * kb);
+                const float dxv[4] = {dx.x, dx.y, dx.z, dx.w};
+                const wf4 ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, mb, wf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int isum = 8 * acc[r][0][i] + acc[r][1][i];
+                    facc[r][i] = fmaf(dxv[i], fmaf(-dmin, ms[i], d * (float)isum), facc[r][i]);
+                }
+            }
+        };
+        for (int b = 0; b < KB; b += 2) {
+            iter(std::integral_constant<int, 0>{}, b);
+            if (b + 1 < KB) iter(std::integral_constant<int, 1>{}, b + 1);
+        }
+        const int n = n0 + 16 * wave + l16;
+#pragma unroll
+        for (int r = 0; r < RL; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int m = 16 * r + 4 * kb + i;
+                if (m < rows && n < N) y[(size_t)(m0 + m) * ldy + n] = facc[r][i];
+            }
+    };
+    switch ((rows + 15) >> 4) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        default: run(std::integral_constant<int, 4>{}); break;
+    }
+}
+
 // ---- Q6_K, wide tiles ----
 // The same skeleton for Q6_K: NW wavefronts side by side in N share 16 RT
 // activation rows, one 16-column tile each, so each weight block is turned
@@ -1208,6 +1377,14 @@ hipError_t launch_grouped_cfg(const uint8_t* w, ActView act, float* y, int max_t
     return hipGetLastError();
 }
 
+hipError_t launch_grouped_wide(const uint8_t* w, ActView act, float* y, int max_tiles, int N, int K, int ldy,
+                               const MmqGroup& g, hipStream_t s) {
+    using T = WideTile<GRP_RT, 1, GRP_NW>;
+    hipLaunchKernelGGL(mmq_q4k_grouped_kernel, dim3(max_tiles, (N + T::BN - 1) / T::BN), dim3(T::NT), 0, s, w, act, y, N,
+                       K, ldy, g);
+    return hipGetLastError();
+}
+
 template <class F>
 hipError_t launch_grouped_fmt(const uint8_t* w, ActView act, float* y, int bm, int max_tiles, int N, int K, int ldy,
                               const MmqGroup& g, hipStream_t s) {
@@ -1409,12 +1586,16 @@ hipError_t launch_mmq(const MmqPlan& plan, int dtype, const uint8_t* w, ActView 
     }
 }
 
-int mmq_group_rows(int rows_per_expert) { return rows_per_expert >= 24 ? 32 : 16; }
+int mmq_group_rows(int dtype, int rows_per_expert, bool wide) {
+    if (dtype == GGML_Q4K && wide && rows_per_expert >= MMQ_GROUP_WIDE_MIN) return MMQ_GROUP_WIDE_ROWS;
+    return rows_per_expert >= 24 ? 32 : 16;
+}
 
 hipError_t launch_mmq_grouped(int dtype, const uint8_t* w, ActView act, float* y, int bm, int max_tiles, int N, int K,
                               int ldy, const MmqGroup& g, hipStream_t s) {
     if (!mmq_supported(dtype) || max_tiles <= 0) return max_tiles == 0 ? hipSuccess : hipErrorInvalidValue;
     if (g.w2 && g.n_split % 64) return hipErrorInvalidValue;  // a column tile must not straddle W | W2
+    if (bm == MMQ_GROUP_WIDE_ROWS) return launch_grouped_wide(w, act, y, max_tiles, N, K, ldy, g, s);
     // (the register-staged kernel: the LDS DMA one measured 4-10% slower on the
     // MoE layer's short K loops)
     if (dtype == GGML_Q4K) return launch_grouped_fmt<MmqQ4K>(w, act, y, bm, max_tiles, N, K, ldy, g, s);

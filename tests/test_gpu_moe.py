@@ -177,6 +177,37 @@ def test_moe_ffn(dev, t, d, ffn, e, k, dt):
     assert err < TOL
 
 
+@pytest.mark.parametrize("d,ffn", [(512, 256), (256, 768)])
+def test_moe_ffn_grouped_tile_edges(dev, d, ffn):
+    """Experts whose row counts sit on the edges of the grouped tiles (16-row
+    parts, 64-row tiles; an expert without rows), one superblock and several;
+    and the same bits from weights off 16-byte alignment, which take the
+    register-staged tiles."""
+    counts = [0, 1, 15, 16, 17, 32, 33, 48, 49, 63, 64, 65, 130, 2, 31, 47]
+    say("moe_ffn grouped tile edges", d, ffn)
+    e = len(counts)
+    pick = np.random.default_rng(d).permutation(np.repeat(np.arange(e), counts))
+    t = pick.size
+    logits = O.normal((t, e), seed=71, stream=2)
+    logits[np.arange(t), pick] += 100.0
+    x = O.normal((t, d), seed=72, stream=1)
+    w = [device_experts(dev, O.Q4K, e, r, c, 73, 3 + i) for i, (r, c) in enumerate([(ffn, d), (ffn, d), (d, ffn)])]
+    ids, wts, *_ = O.moe_route(logits, 1)
+    assert np.array_equal(np.bincount(ids[:, 0], minlength=e), counts)
+    want = O.moe_ffn(O.Q4K, x, ids, wts, *(b for _, b in w))
+    xd, ld = dev.from_numpy(x), dev.from_numpy(logits)
+    got = F.moe_ffn(dev, O.Q4K, xd, ld, *(q for q, _ in w), ffn, 1).numpy()
+    for i in range(e):  # (row by row: one wrong row of many would hide in the norm)
+        rows = np.nonzero(pick == i)[0]
+        assert all(rel_err(got[r], want[r]) < TOL for r in rows), counts[i]
+    shifted = []
+    for _, b in w:
+        raw = np.concatenate([np.zeros(4, np.uint8), np.frombuffer(b.tobytes(), np.uint8)])
+        shifted.append(dev.from_numpy(raw))
+    off = F.moe_ffn(dev, O.Q4K, xd, ld, *(s.ptr + 4 for s in shifted), ffn, 1).numpy()
+    assert off.tobytes() == got.tobytes()
+
+
 def test_moe_ffn_errors(dev):
     x = dev.alloc((2, 256), np.float32)
     logits = dev.alloc((2, 4), np.float32)
