@@ -109,6 +109,18 @@ struct Q80Wave {
     uint16_t dbits;
 };
 
+// The SoA workspace entries of superblock sb (row m's superblock b: sb = m K /
+// 256 + b).
+__device__ __forceinline__ void q8k_store(const Q8KWave& r, const ActView& act, size_t sb, int lane) {
+    reinterpret_cast<uint32_t*>(act.qs + sb * QK_K)[lane] = r.packed;
+    if ((lane & 3) == 0) {
+        act.bsums[sb * 16 + (lane >> 2)] = (int16_t)r.bsum;
+        // (|bsum| <= 2032: exact in f16)
+        if (act.bsh) act.bsh[sb * 16 + (lane >> 2)] = __builtin_bit_cast(uint16_t, (_Float16)(float)r.bsum);
+    }
+    if (lane == 0) act.d[sb] = r.d;
+}
+
 // `v` = elements 4*(lane%8).. of block lane/8 (zeros for lanes without a block).
 __device__ __forceinline__ Q80Wave q8_0_quantize_vals(const float4 v, int lane) {
     const float xv[4] = {v.x, v.y, v.z, v.w};

@@ -6,19 +6,20 @@
 
 namespace frq {
 
-// One wavefront per 256-element superblock; grid = (K/256, rows).  Writes the
-// SoA workspace and, if aos != nullptr, fuel's BlockQ8K bytes.
-__global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restrict__ x, int ldx, int K,
-                                                          ActView act, uint8_t* __restrict__ aos) {
-    const int b = blockIdx.x, m = blockIdx.y, lane = threadIdx.x;
+// The Q8K kernels: one wavefront per 256-element superblock, four of a row a
+// workgroup (one-wavefront workgroups were bound by their launch: 512 rows of
+// 4096 6.6 -> FIGQ us, 4096 rows of silu(g) * u over 768 9.9 -> FIGS);
+// grid = (ceil(K / 1024), rows).
+constexpr int QZ_NW = 4;
+
+// Writes the SoA workspace and, if aos != nullptr, fuel's BlockQ8K bytes.
+__global__ __launch_bounds__(64 * QZ_NW) void quantize_q8k_kernel(const float* __restrict__ x, int ldx, int K,
+                                                                  ActView act, uint8_t* __restrict__ aos) {
+    const int b = blockIdx.x * QZ_NW + (threadIdx.x >> 6), m = blockIdx.y, lane = threadIdx.x & 63;
     const int KB = K / QK_K;
+    if (b >= KB) return;  // (whole wavefronts)
     const Q8KWave r = q8k_quantize_wave(x + (size_t)m * ldx + (size_t)b * QK_K, lane);
-    reinterpret_cast<uint32_t*>(act.qs + (size_t)m * K + (size_t)b * QK_K)[lane] = r.packed;
-    if ((lane & 3) == 0) {
-        act.bsums[((size_t)m * KB + b) * 16 + (lane >> 2)] = (int16_t)r.bsum;
-        if (act.bsh) act.bsh[((size_t)m * KB + b) * 16 + (lane >> 2)] = f32_to_f16_rne((float)r.bsum);
-    }
-    if (lane == 0) act.d[(size_t)m * KB + b] = r.d;
+    q8k_store(r, act, (size_t)m * (K / QK_K) + b, lane);
     if (aos) {
         uint8_t* blk = aos + ((size_t)m * KB + b) * Q8K_BYTES;
         reinterpret_cast<uint32_t*>(blk + 4)[lane] = r.packed;
@@ -28,41 +29,32 @@ __global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restric
 }
 
 // f16 rows (matmul_f16): each half widened exactly to f32, then the same
-// from_float as above; grid = (K/256, rows).
-__global__ __launch_bounds__(64) void quantize_q8k_h_kernel(const uint16_t* __restrict__ x, int K, ActView act) {
-    const int b = blockIdx.x, m = blockIdx.y, lane = threadIdx.x;
-    const int KB = K / QK_K;
+// from_float as above.
+__global__ __launch_bounds__(64 * QZ_NW) void quantize_q8k_h_kernel(const uint16_t* __restrict__ x, int K,
+                                                                    ActView act) {
+    const int b = blockIdx.x * QZ_NW + (threadIdx.x >> 6), m = blockIdx.y, lane = threadIdx.x & 63;
+    if (b >= K / QK_K) return;
     const uint2 h = reinterpret_cast<const uint2*>(x + (size_t)m * K + (size_t)b * QK_K)[lane];
     const float4 v = make_float4(f16_to_f32(h.x & 0xffffu), f16_to_f32(h.x >> 16), f16_to_f32(h.y & 0xffffu),
                                  f16_to_f32(h.y >> 16));
     const Q8KWave r = q8k_quantize_vals(v, lane);
-    reinterpret_cast<uint32_t*>(act.qs + (size_t)m * K + (size_t)b * QK_K)[lane] = r.packed;
-    if ((lane & 3) == 0) {
-        act.bsums[((size_t)m * KB + b) * 16 + (lane >> 2)] = (int16_t)r.bsum;
-        if (act.bsh) act.bsh[((size_t)m * KB + b) * 16 + (lane >> 2)] = f32_to_f16_rne((float)r.bsum);
-    }
-    if (lane == 0) act.d[(size_t)m * KB + b] = r.d;
+    q8k_store(r, act, (size_t)m * (K / QK_K) + b, lane);
 }
 
 // SwiGLU input of the down projection: rows of silu(g) * u, g rows in x and
-// u rows in x2 (both of row stride ldx); grid = (K/256, rows).
-__global__ __launch_bounds__(64) void quantize_q8k_swiglu_kernel(const float* __restrict__ x,
-                                                                 const float* __restrict__ x2, int ldx, int K,
-                                                                 ActView act) {
-    const int b = blockIdx.x, m = blockIdx.y, lane = threadIdx.x;
-    const int KB = K / QK_K;
+// u rows in x2 (both of row stride ldx).
+__global__ __launch_bounds__(64 * QZ_NW) void quantize_q8k_swiglu_kernel(const float* __restrict__ x,
+                                                                         const float* __restrict__ x2, int ldx, int K,
+                                                                         ActView act) {
+    const int b = blockIdx.x * QZ_NW + (threadIdx.x >> 6), m = blockIdx.y, lane = threadIdx.x & 63;
+    if (b >= K / QK_K) return;
     const size_t o = (size_t)m * ldx + (size_t)b * QK_K;
     const float4 gv = reinterpret_cast<const float4*>(x + o)[lane];
     const float4 uv = reinterpret_cast<const float4*>(x2 + o)[lane];
     const float4 h = make_float4(silu_mul(gv.x, uv.x), silu_mul(gv.y, uv.y), silu_mul(gv.z, uv.z),
                                  silu_mul(gv.w, uv.w));
     const Q8KWave r = q8k_quantize_vals(h, lane);
-    reinterpret_cast<uint32_t*>(act.qs + (size_t)m * K + (size_t)b * QK_K)[lane] = r.packed;
-    if ((lane & 3) == 0) {
-        act.bsums[((size_t)m * KB + b) * 16 + (lane >> 2)] = (int16_t)r.bsum;
-        if (act.bsh) act.bsh[((size_t)m * KB + b) * 16 + (lane >> 2)] = f32_to_f16_rne((float)r.bsum);
-    }
-    if (lane == 0) act.d[(size_t)m * KB + b] = r.d;
+    q8k_store(r, act, (size_t)m * (K / QK_K) + b, lane);
 }
 
 // Rows of rms_norm(x) * gain quantized to Q8K: one workgroup of QR_NW
@@ -94,12 +86,7 @@ __global__ __launch_bounds__(64 * QR_NW) void quantize_q8k_rms_kernel(const floa
         const int b = w + QR_NW * i;
         if (b >= KB) break;
         const Q8KWave r = q8k_quantize_vals(pre.v[i], lane);
-        reinterpret_cast<uint32_t*>(act.qs + (size_t)m * K + (size_t)b * QK_K)[lane] = r.packed;
-        if ((lane & 3) == 0) {
-            act.bsums[((size_t)m * KB + b) * 16 + (lane >> 2)] = (int16_t)r.bsum;
-            if (act.bsh) act.bsh[((size_t)m * KB + b) * 16 + (lane >> 2)] = f32_to_f16_rne((float)r.bsum);
-        }
-        if (lane == 0) act.d[(size_t)m * KB + b] = r.d;
+        q8k_store(r, act, (size_t)m * (K / QK_K) + b, lane);
     }
 }
 
@@ -148,22 +135,23 @@ hipError_t launch_quantize_q8_0_h(const uint16_t* x, int rows, int K, ActView ac
     return hipGetLastError();
 }
 
+static dim3 q8k_grid(int K, int rows) { return dim3((K / QK_K + QZ_NW - 1) / QZ_NW, rows); }
+
 hipError_t launch_quantize_q8k(const float* x, int rows, int K, ActView act, uint8_t* aos,
                                hipStream_t s) {
-    dim3 grid(K / QK_K, rows);
-    hipLaunchKernelGGL(quantize_q8k_kernel, grid, dim3(64), 0, s, x, K, K, act, aos);
+    hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(64 * QZ_NW), 0, s, x, K, K, act, aos);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_q8k_h(const uint16_t* x, int rows, int K, ActView act, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(quantize_q8k_h_kernel, dim3(K / QK_K, rows), dim3(64), 0, s, x, K, act);
+    hipLaunchKernelGGL(quantize_q8k_h_kernel, q8k_grid(K, rows), dim3(64 * QZ_NW), 0, s, x, K, act);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_q8k_swiglu(const float* x, int ldx, int rows, int K, ActView act, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(quantize_q8k_swiglu_kernel, dim3(K / QK_K, rows), dim3(64), 0, s, x, x + K, ldx, K, act);
+    hipLaunchKernelGGL(quantize_q8k_swiglu_kernel, q8k_grid(K, rows), dim3(64 * QZ_NW), 0, s, x, x + K, ldx, K, act);
     return hipGetLastError();
 }
 
@@ -175,8 +163,8 @@ hipError_t launch_quantize_q8k_src(const ActSrc& src, int rows, int K, ActView a
     if (rows <= 0) return hipSuccess;
     if (!quantize_src_supported(src, K)) return hipErrorInvalidValue;
     if (src.x2) {
-        hipLaunchKernelGGL(quantize_q8k_swiglu_kernel, dim3(K / QK_K, rows), dim3(64), 0, s, src.x, src.x2, src.ldx,
-                           K, act);
+        hipLaunchKernelGGL(quantize_q8k_swiglu_kernel, q8k_grid(K, rows), dim3(64 * QZ_NW), 0, s, src.x, src.x2,
+                           src.ldx, K, act);
     } else if (src.gain) {
         const int maxq = (K / QK_K + QR_NW - 1) / QR_NW;
 #define FRQ_QR(q)                                                                                                 \
@@ -190,7 +178,7 @@ hipError_t launch_quantize_q8k_src(const ActSrc& src, int rows, int K, ActView a
         }
 #undef FRQ_QR
     } else {
-        hipLaunchKernelGGL(quantize_q8k_kernel, dim3(K / QK_K, rows), dim3(64), 0, s, src.x, src.ldx, K, act,
+        hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(64 * QZ_NW), 0, s, src.x, src.ldx, K, act,
                            (uint8_t*)nullptr);
     }
     return hipGetLastError();
