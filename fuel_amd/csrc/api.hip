@@ -484,11 +484,10 @@ int check_moe_dims(const char* who, size_t e, size_t topk) {
 // Routing + expert batches into caller buffers; entry_expert / entry_pos are
 // device scratch of t * topk ints.
 int route_and_batch(frq_device* dev, const float* logits, size_t t, size_t e, size_t topk, int* ids, float* w,
-                    int* offsets, int* sorted_token, int* sorted_slot, int* entry_expert, int* entry_pos,
-                    const MoeTiles& tiles = MoeTiles{}) {
+                    int* offsets, int* sorted_token, int* sorted_slot, int* entry_expert, int* entry_pos) {
     HIP_TRY(launch_moe_route(logits, (int)t, (int)e, (int)topk, ids, w, dev->stream));
     HIP_TRY(launch_moe_batches(ids, (int)(t * topk), (int)e, (int)topk, offsets, sorted_token, sorted_slot,
-                               entry_expert, entry_pos, tiles, dev->stream));
+                               entry_expert, entry_pos, MoeTiles{}, dev->stream));
     return FRQ_OK;
 }
 
@@ -1055,18 +1054,18 @@ int frq_moe_ffn(frq_device* dev, int dt, size_t t, size_t d, size_t ffn, size_t 
     // launch rows in (token, slot) order straight from the routing, and the
     // combine still sums each token's entries in ascending expert order.
     if (grouped) {
-        if ((rc = route_and_batch(dev, logits, t, e, topk, ids, wts, offsets, sorted_token, nullptr, entry_expert,
-                                  entry_pos, tiles)))
-            return rc;
+        // the routing and the x rows quantized once; the gate|up tiles gather them by token
+        HIP_TRY(launch_moe_route_quantize(logits, (int)t, (int)e, (int)topk, ids, wts, x, (int)d,
+                                          act_view(ax, GGML_Q8K, t, d), dev->stream));
+        HIP_TRY(launch_moe_batches(ids, (int)p, (int)e, (int)topk, offsets, sorted_token, nullptr, entry_expert,
+                                   entry_pos, tiles, dev->stream));
     } else if (e > (size_t)QMV_ROUTE_MAX_EXPERTS) {  // (with fewer experts the gate|up launch routes)
         HIP_TRY(launch_moe_route(logits, (int)t, (int)e, (int)topk, ids, wts, dev->stream));
     }
     const size_t gate_bytes = ffn * (d / bs) * type_size(dt);
     const size_t down_bytes = d * (ffn / bs) * type_size(dt);
     if (grouped) {
-        // x rows quantized once; the gate|up tiles gather them by token
         const ActView xv = act_view(ax, GGML_Q8K, t, d);
-        HIP_TRY(launch_quantize_q8k(x, (int)t, (int)d, xv, nullptr, dev->stream));
         MmqGroup g{};
         g.tile_expert = tiles.tile_expert;
         g.tile_row0 = tiles.tile_row0;

@@ -117,6 +117,9 @@ hipError_t launch_qmv_pair(int dt1, const uint8_t* w1, float* y1, int n1, int dt
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_MAX_TOPK = 64;
 hipError_t launch_moe_route(const float* logits, int T, int E, int topk, int* ids, float* w, hipStream_t s);
+// The same and the Q8K rows of x [T, K], in one launch.
+hipError_t launch_moe_route_quantize(const float* logits, int T, int E, int topk, int* ids, float* w, const float* x,
+                                     int K, ActView act, hipStream_t s);
 // With tile_bm > 0 the batches kernel also writes the tile table of a grouped
 // matmul: tiles of tile_bm sorted rows, expert by expert (tile_expert,
 // tile_row0, ntiles[0] = count; at most P / tile_bm + E tiles).

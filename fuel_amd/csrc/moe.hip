@@ -46,6 +46,38 @@ __global__ __launch_bounds__(ROUTE_WG) void moe_route_kernel(const float* __rest
     }
 }
 
+// The routing and the Q8K quantize of the token rows in one launch, which do not
+// depend on each other: workgroups 0 .. nroute - 1 route four tokens each, the
+// others quantize four superblocks each (superblock t of row m: t = m K / 256 +
+// b).  512 tokens, 128 experts, 2048 columns: 6.2 + 5.1 us as two launches,
+// 7.0 in one.
+template <int EPL>
+__global__ __launch_bounds__(ROUTE_WG) void moe_route_quantize_kernel(const float* __restrict__ logits, int T, int E,
+                                                                     int topk, int* __restrict__ ids,
+                                                                     float* __restrict__ wts, int nroute,
+                                                                     const float* __restrict__ x, int K, ActView act) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if ((int)blockIdx.x < nroute) {
+        const int t = blockIdx.x * (ROUTE_WG / 64) + wave;
+        if (t >= T) return;  // whole wavefront
+        RouteRow<EPL> row;
+        route_load<EPL>(logits + (size_t)t * E, E, lane, row);
+        int id;
+        float wv;
+        route_topk<EPL>(row, E, topk, lane, id, wv);
+        if (lane < topk) {
+            ids[(size_t)t * topk + lane] = id;
+            wts[(size_t)t * topk + lane] = wv;
+        }
+        return;
+    }
+    const int KB = K / QK_K;
+    const size_t sb = (size_t)((int)blockIdx.x - nroute) * (ROUTE_WG / 64) + wave;
+    if (sb >= (size_t)T * KB) return;
+    // (the rows are contiguous, so superblock sb of all starts at 256 sb)
+    q8k_store(q8k_quantize_wave(x + sb * QK_K, lane), act, sb, lane);
+}
+
 // ---- expert batches ----
 
 constexpr int BATCH_WG = 1024;
@@ -155,120 +187,108 @@ __global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __rest
     }
 }
 
-// The same batches for E <= 256 experts, ranked with ballots instead of
-// bitmaps (measured: 23-29 us -> a few us for 4096 entries).  The entries go in
-// rounds of BATCH_NW * 64 * BATCH_G; wavefront w of a round takes BATCH_G
-// consecutive 64-entry groups.  Within a group, the lanes holding an entry of
-// the same expert are found by eight ballots over the id's bits (the lanes
-// that agree on every bit), so an entry's rank among them is a popcount below
-// its lane; the wavefront's running count per expert (LDS) turns that into a
-// rank within the wavefront's share of the round.  Then, per expert, an
-// exclusive prefix over the wavefronts (plus the earlier rounds' entries)
-// places every entry: (round, wavefront, group, lane) is entry order, so
-// (token, slot) order within an expert is kept, as build_expert_batches does.
-constexpr int BATCH_NW = BATCH_WG / 64;
-constexpr int BATCH_G = 4;
-constexpr int BALLOT_MAX_EXPERTS = 256;
+// The same batches for E <= 256 experts: workgroup c places the entries of chunk
+// c (per of them, a multiple of 256; at most 256 chunks) on its own.  It counts all P entries per expert (LDS
+// adds: the totals give every expert's offset and tiles) and those before its
+// chunk; within the chunk, the lanes of a wavefront holding the same expert are
+// found by eight ballots over the id's bits (the lanes that agree on every
+// bit), and the wavefronts' counts are summed in order, so entries keep their
+// (token, slot) order within an expert, as build_expert_batches does.
+// Workgroup 0 also writes the offsets and the tile table.  One workgroup
+// walking the chunks took 12.5 us for 4096 entries (a chain of barriers on one
+// CU); every workgroup reading all ids again takes 5.9 us.
+constexpr int RANK_WG = 256, RANK_NW = RANK_WG / 64;
+constexpr int RANK_MAX_EXPERTS = 256;
 
-__global__ __launch_bounds__(BATCH_WG) void moe_batches_ballot_kernel(const int* __restrict__ ids, int P, int E,
-                                                                     int topk, int* __restrict__ offsets,
-                                                                     int* __restrict__ sorted_token,
-                                                                     int* __restrict__ sorted_slot,
-                                                                     int* __restrict__ entry_expert,
-                                                                     int* __restrict__ entry_pos, MoeTiles tiles) {
-    __shared__ int off[BALLOT_MAX_EXPERTS];
-    __shared__ int fill[BALLOT_MAX_EXPERTS];
-    __shared__ int wcnt[BATCH_NW][BALLOT_MAX_EXPERTS];
-    __shared__ int wsum[BATCH_NW];
+__global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __restrict__ ids, int P, int E, int topk,
+                                                                   int per, int* __restrict__ offsets,
+                                                                   int* __restrict__ sorted_token,
+                                                                   int* __restrict__ sorted_slot,
+                                                                   int* __restrict__ entry_expert,
+                                                                   int* __restrict__ entry_pos, MoeTiles tiles) {
+    __shared__ int tot[RANK_MAX_EXPERTS], bef[RANK_MAX_EXPERTS];
+    __shared__ int wcnt[RANK_NW][RANK_MAX_EXPERTS];
+    __shared__ int wsum[RANK_NW], tsum[RANK_NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-    // counts -> expert_offsets (and the tile table), as moe_batches_kernel
-    for (int e = tid; e < E; e += BATCH_WG) {
-        off[e] = 0;
-        fill[e] = 0;
+    const int c0 = blockIdx.x * per, c1 = min(P, c0 + per);
+    tot[tid] = 0;  // (RANK_MAX_EXPERTS == RANK_WG)
+    bef[tid] = 0;
+    __syncthreads();
+    constexpr int UN = 8;
+    for (int b0 = 0; b0 < P; b0 += UN * RANK_WG) {
+        int v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const int q = b0 + u * RANK_WG + tid;
+            v[u] = q < P ? ids[q] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if ((unsigned)v[u] < (unsigned)E) {
+                atomicAdd(&tot[v[u]], 1);
+                if (b0 + u * RANK_WG < c0) atomicAdd(&bef[v[u]], 1);  // (an earlier chunk)
+            }
     }
     __syncthreads();
-    for (int i = tid; i < P; i += BATCH_WG) {
-        const int e = ids[i];
-        if ((unsigned)e < (unsigned)E) atomicAdd(&off[e], 1);
+    // exclusive scans over the experts (one a thread) of the counts and the tiles
+    const int c = tid < E ? tot[tid] : 0;
+    const int nt = tiles.bm > 0 ? (c + tiles.bm - 1) / tiles.bm : 0;
+    const int incl = wave_incl_scan(c, lane), tincl = wave_incl_scan(nt, lane);
+    if (lane == 63) {
+        wsum[wave] = incl;
+        tsum[wave] = tincl;
     }
     __syncthreads();
-    const int c = tid < E ? off[tid] : 0;
-    const int incl = wave_incl_scan(c, lane);
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < wave; w++) base += wsum[w];
+    int base = 0, tbase = 0;
+    for (int w = 0; w < wave; w++) {
+        base += wsum[w];
+        tbase += tsum[w];
+    }
     const int excl = base + incl - c;
-    if (tid < E) {
-        off[tid] = excl;
-        offsets[tid] = excl;
-    }
-    if (tid == E - 1) offsets[E] = excl + c;
-    if (tiles.bm > 0) {
-        const int nt = (c + tiles.bm - 1) / tiles.bm;
-        const int tincl = wave_incl_scan(nt, lane);
-        __syncthreads();
-        if (lane == 63) wsum[wave] = tincl;
-        __syncthreads();
-        int tbase = 0;
-        for (int w = 0; w < wave; w++) tbase += wsum[w];
-        const int t0 = tbase + tincl - nt;
-        for (int j = 0; j < nt; j++) {
-            tiles.tile_expert[t0 + j] = tid;
-            tiles.tile_row0[t0 + j] = excl + j * tiles.bm;
-        }
-        if (tid == E - 1) tiles.ntiles[0] = t0 + nt;
-    }
-    __syncthreads();
-
-    const unsigned long long below = (1ull << lane) - 1ull;
-    constexpr int ROUND = BATCH_NW * 64 * BATCH_G;
-    for (int r0 = 0; r0 < P; r0 += ROUND) {
-        for (int e = lane; e < E; e += 64) wcnt[wave][e] = 0;  // (this wavefront's row only)
-        const int g0 = r0 + wave * 64 * BATCH_G;
-        int ee[BATCH_G], rk[BATCH_G];
-#pragma unroll
-        for (int g = 0; g < BATCH_G; g++) {
-            const int i = g0 + 64 * g + lane;
-            const int e = i < P ? ids[i] : -1;
-            const bool valid = (unsigned)e < (unsigned)E;
-            unsigned long long m = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const bool bit = (e >> b) & 1;
-                const unsigned long long v = __ballot(bit);
-                m &= bit ? v : ~v;
+    bef[tid] += excl;  // where the chunk's first entry of expert tid goes
+    if (blockIdx.x == 0) {
+        if (tid < E) offsets[tid] = excl;
+        if (tid == E - 1) offsets[E] = excl + c;
+        if (tiles.bm > 0) {
+            const int t0 = tbase + tincl - nt;
+            for (int j = 0; j < nt; j++) {
+                tiles.tile_expert[t0 + j] = tid;
+                tiles.tile_row0[t0 + j] = excl + j * tiles.bm;
             }
-            const int rank = __popcll(m & below);
-            const int before = valid ? wcnt[wave][e] : 0;
-            if (valid && rank == 0) wcnt[wave][e] = before + __popcll(m);
-            ee[g] = valid ? e : -1;
-            rk[g] = before + rank;
+            if (tid == E - 1) tiles.ntiles[0] = t0 + nt;
         }
-        __syncthreads();
-        for (int e = tid; e < E; e += BATCH_WG) {  // prefix over the wavefronts, after the earlier rounds
-            int run = fill[e];
-            for (int w = 0; w < BATCH_NW; w++) {
-                const int cw = wcnt[w][e];
-                wcnt[w][e] = run;
-                run += cw;
-            }
-            fill[e] = run;
-        }
-        __syncthreads();
+    }
+    for (int i0 = c0; i0 < c1; i0 += RANK_WG) {
 #pragma unroll
-        for (int g = 0; g < BATCH_G; g++) {
-            const int e = ee[g];
-            if (e < 0) continue;
-            const int i = g0 + 64 * g + lane;
-            const int pos = off[e] + wcnt[wave][e] + rk[g];
+        for (int w = 0; w < RANK_NW; w++) wcnt[w][tid] = 0;
+        __syncthreads();
+        const int i = i0 + tid;
+        const int e = i < c1 ? ids[i] : -1;
+        const bool valid = (unsigned)e < (unsigned)E;
+        // rank among the wavefront's entries of the same expert
+        unsigned long long m = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const bool bit = (e >> b) & 1;
+            const unsigned long long v = __ballot(bit);
+            m &= bit ? v : ~v;
+        }
+        const int rank = __popcll(m & ((1ull << lane) - 1ull));
+        if (valid && rank == 0) wcnt[wave][e] = __popcll(m);
+        __syncthreads();
+        if (valid) {
+            int pos = bef[e] + rank;
+            for (int w = 0; w < wave; w++) pos += wcnt[w][e];
             sorted_token[pos] = i / topk;
             if (sorted_slot) sorted_slot[pos] = i;
             entry_expert[pos] = e;
             entry_pos[i] = pos;
         }
         __syncthreads();
+        if (i0 + RANK_WG < c1) {
+#pragma unroll
+            for (int w = 0; w < RANK_NW; w++) bef[tid] += wcnt[w][tid];
+        }
     }
 }
 
@@ -589,12 +609,33 @@ hipError_t launch_moe_route(const float* logits, int T, int E, int topk, int* id
     return hipGetLastError();
 }
 
+hipError_t launch_moe_route_quantize(const float* logits, int T, int E, int topk, int* ids, float* w, const float* x,
+                                     int K, ActView act, hipStream_t s) {
+    if (T <= 0) return hipSuccess;
+    constexpr int PER = ROUTE_WG / 64;
+    const int nroute = (T + PER - 1) / PER;
+    const dim3 grid((unsigned)(nroute + ((size_t)T * (K / QK_K) + PER - 1) / PER));
+#define FRQ_RQ(epl)                                                                                                  \
+    hipLaunchKernelGGL(moe_route_quantize_kernel<epl>, grid, dim3(ROUTE_WG), 0, s, logits, T, E, topk, ids, w, nroute, \
+                       x, K, act)
+    if (E <= 64) FRQ_RQ(1);
+    else if (E <= 128) FRQ_RQ(2);
+    else if (E <= 256) FRQ_RQ(4);
+    else if (E <= 512) FRQ_RQ(8);
+    else if (E <= MOE_MAX_EXPERTS) FRQ_RQ(16);
+    else return hipErrorInvalidValue;
+#undef FRQ_RQ
+    return hipGetLastError();
+}
+
 hipError_t launch_moe_batches(const int* ids, int P, int E, int topk, int* offsets, int* sorted_token,
                               int* sorted_slot, int* entry_expert, int* entry_pos, const MoeTiles& tiles,
                               hipStream_t s) {
     if (E <= 0 || E > MOE_MAX_EXPERTS || topk <= 0) return hipErrorInvalidValue;
-    if (E <= BALLOT_MAX_EXPERTS) {
-        hipLaunchKernelGGL(moe_batches_ballot_kernel, dim3(1), dim3(BATCH_WG), 0, s, ids, P, E, topk, offsets,
+    if (E <= RANK_MAX_EXPERTS) {
+        const int groups = (P + RANK_WG - 1) / RANK_WG, per = RANK_WG * ((groups + 255) / 256);
+        const int wgs = P > 0 ? (P + per - 1) / per : 1;  // (no entries: the offsets all the same)
+        hipLaunchKernelGGL(moe_batches_rank_kernel, dim3(wgs), dim3(RANK_WG), 0, s, ids, P, E, topk, per, offsets,
                            sorted_token, sorted_slot, entry_expert, entry_pos, tiles);
         return hipGetLastError();
     }

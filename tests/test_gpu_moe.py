@@ -54,7 +54,9 @@ def test_moe_route_known_answer(dev):
 
 
 @pytest.mark.parametrize("t,e,k", [(1, 128, 8), (16, 128, 8), (512, 128, 8), (37, 64, 1), (9, 300, 20),
-                                   (3, 1000, 64), (2000, 128, 8)])
+                                   (3, 1000, 64), (2000, 128, 8),
+                                   # batches of one chunk more and less than a workgroup, and of several rounds a chunk
+                                   (32, 256, 8), (33, 255, 8), (257, 200, 1), (9000, 40, 8)])
 def test_moe_route_bit_exact(dev, t, e, k):
     say("moe_route", t, e, k)
     logits = O.normal((t, e), seed=t * 1000 + e, stream=7)
