@@ -18,9 +18,9 @@
 // its 8-term dot products on the VALU.)  f32 step: y += d_x*(d*isum - dmin*msum).
 //
 // Q6_K.  w_e = (q6_e - 32) * sc_g, with sc_g the int8 scale of 16-element
-// group g, lies in [-4096, 4064]: split w = 128*wh + wl with wl = w & 127 in
-// [0, 127] and wh = w >> 7 (arithmetic) in [-32, 31], both bytes, so
-//   isum = 128 * (X . Wh) + (X . Wl)
+// group g, lies in [-4096, 4064]: split w = 256*wh + wl with wl in [-128, 127]
+// and wh in [-16, 16], both signed bytes, so
+//   isum = 256 * (X . Wh) + (X . Wl)
 // is two exact int8 GEMMs.  The products are formed two per 16-bit lane with
 // one packed multiply-add.  f32 step: y += d_x * (d * isum).
 //
@@ -129,8 +129,8 @@ struct MmqQ6K {
         const uint32_t ls = 4u * (uint32_t)(t & 1);                   // compile-time
         const uint32_t hs = 4u * (uint32_t)(t & 1) + 2u * (uint32_t)(kb >> 1);
         const int sc = (int)(int8_t)((h.sc[t] >> (8 * kb)) & 0xffu);
-        const uint32_t f = (uint32_t)sc & 0xffffu, cst = (uint32_t)(-32 * sc) & 0xffffu;
-        const uint32_t sc16 = f | (f << 16), c16 = cst | (cst << 16);
+        uint32_t sc16, c16;
+        q6_factors(sc, sc16, c16);
         const uint32_t l4[4] = {ql.x, ql.y, ql.z, ql.w}, h4[4] = {qh.x, qh.y, qh.z, qh.w};
         int wl[4], wh[4];
 #pragma unroll
@@ -147,7 +147,7 @@ struct MmqQ6K {
         }
     }
     __device__ static float finish(const v4i (&a)[NACC], int i, const Hdr& h) {
-        const int isum = 128 * a[0][i] + a[1][i];
+        const int isum = 256 * a[0][i] + a[1][i];
         return h.d * (float)isum;
     }
 };

@@ -8,7 +8,7 @@ namespace frq {
 
 // The Q8K kernels: one wavefront per 256-element superblock, four of a row a
 // workgroup (one-wavefront workgroups were bound by their launch: 512 rows of
-// 4096 6.6 -> FIGQ us, 4096 rows of silu(g) * u over 768 9.9 -> FIGS);
+// 4096 6.6 -> 5.9 us, 4096 rows of silu(g) * u over 768 9.9 -> 8.9);
 // grid = (ceil(K / 1024), rows).
 constexpr int QZ_NW = 4;
 

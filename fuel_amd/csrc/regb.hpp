@@ -102,8 +102,8 @@ struct SkQ6K {
         for (int t = 0; t < 4; t++) {  // code t: ql nibble t>>1 of la (t even) / lb (t odd), qh bits 2t
             const uint32_t scw = t < 2 ? r.sc.x : r.sc.y;
             const int sc = (int)(int8_t)((scw >> (16u * (uint32_t)(t & 1) + sel)) & 0xffu);  // scales[8hh + 2t + (c&1)]
-            const uint32_t f = (uint32_t)sc & 0xffffu, cst = (uint32_t)(-32 * sc) & 0xffffu;
-            const uint32_t sc16 = f | (f << 16), c16 = cst | (cst << 16);
+            uint32_t sc16, c16;
+            q6_factors(sc, sc16, c16);
             const uint32_t* l = (t & 1) ? lb : la;
             int wl[4], wh[4];
 #pragma unroll
@@ -125,7 +125,7 @@ struct SkQ6K {
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int isum = 128 * acc[rt][0][i] + acc[rt][1][i];
+                const int isum = 256 * acc[rt][0][i] + acc[rt][1][i];
                 facc[rt][i] = fmaf(dx[rt][i], d * (float)isum, facc[rt][i]);
             }
     }
