@@ -1416,6 +1416,9 @@ enum MmqKind {
     MMQ_Q4K_WIDE16_KG2,  // 16 x 64, two groups of four wavefronts
     MMQ_Q6K_WIDE16,      // 16 x 64, the Q6_K wide-tile kernel with four wavefronts
     MMQ_Q6K_WIDE32,      // 32 x 64, the same
+    MMQ_Q4K_16X32_KG2,   // 16 x 32, two groups of two wavefronts splitting K
+    MMQ_Q4K_32X32_KG2,   // 32 x 32, two groups of two
+    MMQ_Q4K_32X48_KG2,   // 32 x 48, two groups of three
 };
 
 #define FRQ_MMQ_KINDS(X)                          \
@@ -1495,6 +1498,16 @@ MmqPlan mmq_plan(int dtype, const void* w, int M, int N, int K, int num_cus, siz
     // reduce included).  The 16 x 64 tiles also take 3-15 rows of >= 8192
     // columns (the caller's row rule): 4096x32000 M = 4 16.3 us, M = 8 16.8,
     // M = 12 17.4 against 27 us for the 32 x 64 plane kernel.
+    // Where those two-group tiles leave CUs idle, the same two groups over fewer
+    // columns give more of them (the sums keep their order, so the bits):
+    // * up to 16 rows 16 x 32 while three per CU hold the grid (4096x8192 M = 8
+    //   10.8 -> 9.5 us, 4096x11008 11.2 -> 10.4, 4096x14336 11.7 -> 10.8,
+    //   4096x22016 15.7 -> 14.0; past that, 4096x32000, 21.9 against 17.6 in
+    //   16 x 64; 16 x 48 10.5, 13.6 and 14.7 at the last three);
+    // * 17-32 rows the narrowest of 32 x 32 and 32 x 48 that fits one per CU,
+    //   since a second one on a few CUs doubles the launch (4096x8192 M = 24
+    //   13.1 -> 10.8 us in 32 x 32; 4096x11008 M = 32 14.1 -> 12.9 in 32 x 48,
+    //   14.3 in 32 x 32).
     if (dma && M >= 2) {
         using T8 = WideTile<4, 1, 8>;
         using T4 = WideTile<2, 1, 4>;
@@ -1513,9 +1526,13 @@ MmqPlan mmq_plan(int dtype, const void* w, int M, int N, int K, int num_cus, siz
                 p.kind = MMQ_Q4K_WIDE32;
                 p.ks = clamp_ks((3 * C + t4 - 1) / t4);
             } else if (M <= 16) {
-                p.kind = MMQ_Q4K_WIDE16_KG2;
+                p.kind = (N + 31) / 32 <= 3 * C ? MMQ_Q4K_16X32_KG2 : MMQ_Q4K_WIDE16_KG2;
+            } else if (t4 > C) {
+                p.kind = MMQ_Q4K_WIDE32;
             } else {
-                p.kind = t4 <= C ? MMQ_Q4K_WIDE32_KG2 : MMQ_Q4K_WIDE32;
+                p.kind = (N + 31) / 32 <= C   ? MMQ_Q4K_32X32_KG2
+                         : (N + 47) / 48 <= C ? MMQ_Q4K_32X48_KG2
+                                              : MMQ_Q4K_WIDE32_KG2;
             }
         } else if (long_rows && M >= 128 && t8 < 4 * C / 5) {
             const int occ = kernel_occupancy<mmq_q4k_wide_kernel<4, 1, 8>, T8::NT>();
@@ -1580,6 +1597,12 @@ hipError_t launch_mmq(const MmqPlan& plan, int dtype, const uint8_t* w, ActView 
             return launch_wide<2, 1, 4, 2>(w, act, y, M, N, K, ldy, s, out_mode, plan.ks, part);
         case MMQ_Q4K_WIDE16_KG2:
             return launch_wide<1, 1, 4, 2>(w, act, y, M, N, K, ldy, s, out_mode, plan.ks, part);
+        case MMQ_Q4K_16X32_KG2:
+            return launch_wide<1, 1, 2, 2>(w, act, y, M, N, K, ldy, s, out_mode, plan.ks, part);
+        case MMQ_Q4K_32X32_KG2:
+            return launch_wide<2, 1, 2, 2>(w, act, y, M, N, K, ldy, s, out_mode, plan.ks, part);
+        case MMQ_Q4K_32X48_KG2:
+            return launch_wide<2, 1, 3, 2>(w, act, y, M, N, K, ldy, s, out_mode, plan.ks, part);
         case MMQ_Q6K_WIDE16: return launch_wide6<1, 4>(w, act, y, M, N, K, ldy, s, out_mode);
         case MMQ_Q6K_WIDE32: return launch_wide6<2, 4>(w, act, y, M, N, K, ldy, s, out_mode);
         default: return hipErrorInvalidValue;

@@ -482,6 +482,28 @@ def test_qmatmul_wide_tiles(dev, dt, m, n, k):
     assert err16 <= TOL_F16
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (5, 8192, 256), (16, 8193, 512), (9, 24576, 768), (16, 24577, 256),         # 16 x 32, then 16 x 64
+    (17, 8192, 256), (32, 8193, 768), (31, 12288, 512), (17, 12289, 1024),      # 32 x 32, 32 x 48, 32 x 64
+    (3, 16385, 4096), (27, 8240, 4096),
+])
+def test_qmatmul_q4k_narrow_tiles(dev, m, n, k):
+    """The tile widths that 3-32 rows pick, at and just past the column counts
+    where the plan changes width (256 CUs); superblocks fewer than, equal to and
+    not a multiple of the two wavefront groups; ragged rows and columns.  Every
+    row against the oracle: exact integer dots, up to 16 superblocks of two f32
+    terms each, so 32 roundings of 2^-24 = 2e-6 of the row's norm."""
+    say("narrow tiles", m, n, k)
+    wq = O.quantize(O.Q4K, O.normal((n, k), seed=61, stream=2, std=0.02))
+    x = O.normal((m, k), seed=62, stream=1)
+    want = O.matmul(O.Q4K, x, wq)
+    w = dev.from_numpy(np.frombuffer(wq.tobytes(), np.uint32))
+    out = dev.from_numpy(np.full((m, n), np.nan, np.float32))
+    F.qmatmul_f32_rocm_wrapper([dev.from_numpy(x), w], [out], F.QMatMulParams(O.Q4K, 1, m, n, k))
+    got = out.numpy()
+    assert max(rel_err(got[r], want[r]) for r in range(m)) < 2e-6
+
+
 @pytest.mark.parametrize("m", [64, 128])
 def test_qmatmul_q4k_weights_off_16_byte_alignment(dev, m):
     """Q4_K blocks at a 4-byte (not 16-byte) aligned address, as a KernelRef
