@@ -15,6 +15,7 @@ import pytest
 import fuel_amd as F
 import oracle as O
 from blockref import rel_err
+from fuel_amd.hiprt import HipRuntime
 
 pytestmark = pytest.mark.gpu
 
@@ -208,6 +209,48 @@ def test_moe_ffn_grouped_tile_edges(dev, d, ffn):
         shifted.append(dev.from_numpy(raw))
     off = F.moe_ffn(dev, O.Q4K, xd, ld, *(s.ptr + 4 for s in shifted), ffn, 1).numpy()
     assert off.tobytes() == got.tobytes()
+
+
+def test_moe_ffn_full_round_of_tiles(dev):
+    """The grid of the grouped tiles is sized for the most tiles the routing can
+    give; its spare workgroups must not keep the working ones waiting.  Eight
+    experts of 4096 x 4096 fill 256 CUs with exactly one round of gate|up tiles
+    (8 x 64, two resident a CU): routing all eight takes at most 8/7 of the time
+    of routing seven, the work's own ratio (the fastest of 20 replays of either;
+    two sets of weights in turn, so that they come from memory)."""
+    e, d, t, topk = 8, 4096, 16, 2
+    say("moe_ffn full round of tiles")
+    hip = HipRuntime()
+    w = [[dev.qzeros(e * d * d, O.Q4K) for _ in range(3)] for _ in range(2)]
+    x = dev.from_numpy(O.normal((t, d), seed=1, stream=1))
+    out = dev.alloc((t, d), np.float32)
+    s = hip.stream_create()
+    e0, e1 = hip.event_create(), hip.event_create()
+    dev.set_stream(s)
+    best = []
+    try:
+        for used in (7, 8):
+            logits = np.zeros((t, e), np.float32)
+            for i in range(t * topk):
+                logits[i // topk, i % used] = 5 + i % topk
+            ld = dev.from_numpy(logits)
+            F.moe_ffn(dev, O.Q4K, x, ld, *w[0], d, topk, out)
+            hip.stream_sync(s)
+            g = hip.capture(s, lambda: [F.moe_ffn(dev, O.Q4K, x, ld, *w[i % 2], d, topk, out) for i in range(4)])
+            times = []
+            for _ in range(22):
+                hip.event_record(e0, s)
+                hip.graph_launch(g, s)
+                hip.event_record(e1, s)
+                hip.event_sync(e1)
+                times.append(hip.elapsed_ms(e0, e1))
+            hip.graph_destroy(g)
+            best.append(min(times[2:]))
+    finally:
+        dev.set_stream(None)
+        hip.stream_destroy(s)
+    say("  7 and 8 experts:", best)
+    assert best[1] <= best[0] * 8 / 7, best
 
 
 def test_moe_ffn_errors(dev):
