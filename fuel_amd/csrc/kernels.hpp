@@ -183,13 +183,15 @@ struct MmqGroup {
     int n_split;
 };
 // Tile height for an average rows-per-expert.  wide: every operand allows the
-// grouped wide-tile kernel (Q4_K blocks at 16-byte aligned bases, a W | W2
-// split that is a multiple of its 128 columns): from two rows per expert on
-// average (128 experts, top-8, 2048 / 768, the whole layer: 32 tokens 99.8 ->
-// 99.1 us, 192 126 -> 117, 256 141 -> 123, 512 181 -> 147, 1024 293 -> 224
-// against the 16- and 32-row tiles; below two the 16-row tiles, 20 tokens 85.8
-// against 88.3).
-constexpr int MMQ_GROUP_WIDE_ROWS = 64, MMQ_GROUP_WIDE_MIN = 2;
+// grouped wide-tile kernel (Q4_K blocks at 16-byte aligned bases), which is
+// taken at any number of rows.  Whole layers against the 16- and 32-row tiles,
+// us: 128 experts, top-8, 2048 / 768: 20 tokens 76 -> 76, 64 tokens 101 -> 93,
+// 512 179 -> 131; 16 experts, top-2, 1024 / 512: 10 tokens 25 -> 22, 64 26 -> 23;
+// 8 experts, top-2, 4096 / 4096: 16 tokens 73 -> 66, 128 130 -> 82; 32 experts,
+// top-4, 4096 / 2048: 20 tokens 109 -> 99, 64 124 -> 107.  Swept from 1.1 to 64
+// rows an expert over 13 shapes (4-200 experts), none was slower by more than
+// the runs differ.
+constexpr int MMQ_GROUP_WIDE_ROWS = 64;
 int mmq_group_rows(int dtype, int rows_per_expert, bool wide);
 hipError_t launch_mmq_grouped(int dtype, const uint8_t* w, ActView act, float* y, int bm, int max_tiles, int N, int K,
                               int ldy, const MmqGroup& g, hipStream_t s);

@@ -1616,7 +1616,7 @@ hipError_t launch_mmq(const MmqPlan& plan, int dtype, const uint8_t* w, ActView 
 }
 
 int mmq_group_rows(int dtype, int rows_per_expert, bool wide) {
-    if (dtype == GGML_Q4K && wide && rows_per_expert >= MMQ_GROUP_WIDE_MIN) return MMQ_GROUP_WIDE_ROWS;
+    if (dtype == GGML_Q4K && wide) return MMQ_GROUP_WIDE_ROWS;
     return rows_per_expert >= 24 ? 32 : 16;
 }
 
