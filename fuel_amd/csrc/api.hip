@@ -1015,7 +1015,7 @@ int frq_moe_ffn(frq_device* dev, int dt, size_t t, size_t d, size_t ffn, size_t 
         return fail(FRQ_MISALIGNED, "moe_ffn: f32 buffers not 4-byte aligned");
     const size_t p = t * topk;
     const bool grouped = mmq_supported(dt) && (double)p > MOE_MMQ_MIN_ROWS_PER_EXPERT * (double)e;
-    const bool wide = (((uintptr_t)w_gate | (uintptr_t)w_up | (uintptr_t)w_down) & 15u) == 0 && ffn % 128 == 0;
+    const bool wide = (((uintptr_t)w_gate | (uintptr_t)w_up | (uintptr_t)w_down) & 15u) == 0;
     const int bm = mmq_group_rows(dt, (int)(p / e), wide);
     const size_t max_tiles = grouped ? (p + bm - 1) / bm + e : 0;
     // workspace: ids, w, sorted token, entry expert, entry position, offsets,

@@ -1623,8 +1623,13 @@ int mmq_group_rows(int dtype, int rows_per_expert, bool wide) {
 hipError_t launch_mmq_grouped(int dtype, const uint8_t* w, ActView act, float* y, int bm, int max_tiles, int N, int K,
                               int ldy, const MmqGroup& g, hipStream_t s) {
     if (!mmq_supported(dtype) || max_tiles <= 0) return max_tiles == 0 ? hipSuccess : hipErrorInvalidValue;
-    if (g.w2 && g.n_split % 64) return hipErrorInvalidValue;  // a column tile must not straddle W | W2
-    if (bm == MMQ_GROUP_WIDE_ROWS) return launch_grouped_wide(w, act, y, max_tiles, N, K, ldy, g, s);
+    // a column tile must not straddle W | W2, and the wide tiles read whole
+    // 16-byte pieces of Q4_K blocks by LDS DMA
+    const bool wide = bm == MMQ_GROUP_WIDE_ROWS;
+    if (g.w2 && g.n_split % (wide ? WideTile<GRP_RT, 1, GRP_NW>::BN : 64)) return hipErrorInvalidValue;
+    if (wide && (dtype != GGML_Q4K || (((uintptr_t)w | (uintptr_t)g.w2 | g.expert_bytes) & 15u)))
+        return hipErrorInvalidValue;
+    if (wide) return launch_grouped_wide(w, act, y, max_tiles, N, K, ldy, g, s);
     // (the register-staged kernel: the LDS DMA one measured 4-10% slower on the
     // MoE layer's short K loops)
     if (dtype == GGML_Q4K) return launch_grouped_fmt<MmqQ4K>(w, act, y, bm, max_tiles, N, K, ldy, g, s);
