@@ -1509,11 +1509,19 @@ MmqPlan mmq_plan(int dtype, const void* w, int M, int N, int K, int num_cus, siz
     // * up to 16 rows 16 x 32 while three per CU hold the grid (4096x8192 M = 8
     //   10.8 -> 9.5 us, 4096x11008 11.2 -> 10.4, 4096x14336 11.7 -> 10.8,
     //   4096x22016 15.7 -> 14.0; past that, 4096x32000, 21.9 against 17.6 in
-    //   16 x 64; 16 x 48 10.5, 13.6 and 14.7 at the last three);
+    //   16 x 64; 16 x 48 10.5, 13.6 and 14.7 at the last three); between one
+    //   and two per CU only from nine superblocks or 10.5 a CU over its tiles,
+    //   since less does not pay for a second round on part of the CUs (whole
+    //   call at M = 8 against 16 x 64: 10240 columns, 256 elements +8%, 768 +8,
+    //   1280 +6, 1792 +4, 2048 0, 2304 -1, 3072 -3, 7936 -8; 14336 columns, 256
+    //   +7, 1280 +3, 1536 -3, 2048 -2; at 8192 and at 20480 columns none longer
+    //   by more than 1% at any length);
     // * 17-32 rows the narrowest of 32 x 32 and 32 x 48 that fits one per CU,
     //   since a second one on a few CUs doubles the launch (4096x8192 M = 24
     //   13.1 -> 10.8 us in 32 x 32; 4096x11008 M = 32 14.1 -> 12.9 in 32 x 48,
-    //   14.3 in 32 x 32).
+    //   14.3 in 32 x 32); 32 x 48 from three superblocks (whole call at 8224 to
+    //   12288 columns, M = 17-32, against 32 x 64: 256 and 512 elements +1 to
+    //   +5%, 768-2048 equal, 4096 -7 to -10, 7936 -8 to -13).
     if (dma && M >= 2) {
         using T8 = WideTile<4, 1, 8>;
         using T4 = WideTile<2, 1, 4>;
@@ -1532,13 +1540,15 @@ MmqPlan mmq_plan(int dtype, const void* w, int M, int N, int K, int num_cus, siz
                 p.kind = MMQ_Q4K_WIDE32;
                 p.ks = clamp_ks((3 * C + t4 - 1) / t4);
             } else if (M <= 16) {
-                p.kind = (N + 31) / 32 <= 3 * C ? MMQ_Q4K_16X32_KG2 : MMQ_Q4K_WIDE16_KG2;
+                const int n32 = (N + 31) / 32;
+                const bool narrow = n32 <= C || (n32 <= 3 * C && (n32 > 2 * C || KB > 8 || 2 * KB * n32 >= 21 * C));
+                p.kind = narrow ? MMQ_Q4K_16X32_KG2 : MMQ_Q4K_WIDE16_KG2;
             } else if (t4 > C) {
                 p.kind = MMQ_Q4K_WIDE32;
             } else {
-                p.kind = (N + 31) / 32 <= C   ? MMQ_Q4K_32X32_KG2
-                         : (N + 47) / 48 <= C ? MMQ_Q4K_32X48_KG2
-                                              : MMQ_Q4K_WIDE32_KG2;
+                p.kind = (N + 31) / 32 <= C             ? MMQ_Q4K_32X32_KG2
+                         : (N + 47) / 48 <= C && KB > 2 ? MMQ_Q4K_32X48_KG2
+                                                        : MMQ_Q4K_WIDE32_KG2;
             }
         } else if (long_rows && M >= 128 && t8 < 4 * C / 5) {
             const int occ = kernel_occupancy<mmq_q4k_wide_kernel<4, 1, 8>, T8::NT>();

@@ -483,7 +483,7 @@ def test_qmatmul_wide_tiles(dev, dt, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (5, 8192, 256), (16, 8193, 512), (9, 24576, 768), (16, 24577, 256),         # 16 x 32, then 16 x 64
+    (5, 8192, 256), (9, 24576, 768), (7, 8193, 2304), (16, 8193, 512), (16, 24577, 256),  # 16 x 32, then 16 x 64
     (17, 8192, 256), (32, 8193, 768), (31, 12288, 512), (17, 12289, 1024),      # 32 x 32, 32 x 48, 32 x 64
     (3, 16385, 4096), (27, 8240, 4096),
 ])
@@ -502,6 +502,49 @@ def test_qmatmul_q4k_narrow_tiles(dev, m, n, k):
     F.qmatmul_f32_rocm_wrapper([dev.from_numpy(x), w], [out], F.QMatMulParams(O.Q4K, 1, m, n, k))
     got = out.numpy()
     assert max(rel_err(got[r], want[r]) for r in range(m)) < 2e-6
+
+
+@pytest.mark.parametrize("m,k", [(5, 2304), (8, 2304), (16, 4096), (17, 768), (32, 1280)])
+def test_qmatmul_q4k_narrow_tiles_keep_the_bits(dev, m, k):
+    """Up to 16 rows 16 x 32 and 16 x 64 tiles, at 17-32 rows 32 x 32, 32 x 48 and
+    32 x 64 ones: the same columns have the same bits whichever width the number
+    of columns picks (one order of the f32 sums)."""
+    import ctypes as C
+    from fuel_amd._native import check, lib
+    say("narrow tiles' bits", m, k)
+    widths = (8192, 16385, 24577) if m <= 16 else (8192, 8209, 12289)
+    n = max(widths)
+    q = dev.qzeros(n * k, O.Q4K)
+    q.quantize(F.fill_normal(dev, (n, k), 63, 2, 0.0, 0.02))
+    x = dev.from_numpy(acts(m, k))
+    kinds = [F.qmatmul_plan(dev, O.Q4K, m, c, k, q.device_ptr())[1] for c in widths]
+    assert len(set(kinds)) == (2 if m <= 16 else 3)
+    got = []
+    for c in widths:
+        y = dev.alloc((m, c), np.float32)
+        check(lib().frq_qmatmul(dev.handle, O.Q4K, 1, m, c, k, C.c_void_p(x.ptr), m * k * 4,
+                                C.c_void_p(q.device_ptr()), c * k // 256 * 144, C.c_void_p(y.ptr), m * c * 4))
+        got.append(y.numpy())
+    for y in got[:-1]:
+        assert np.array_equal(y.view(np.uint32), got[-1][:, :y.shape[1]].view(np.uint32))
+
+
+def test_qmatmul_q4k_narrow_tiles_where_they_pay(dev):
+    """Between one and two 16 x 32 tiles a CU (8193-16384 columns on 256 CUs), short
+    rows keep the 16 x 64 tiles, which are up to 8% faster there: up to eight
+    superblocks just past one tile a CU, up to five at two.  Rows of one or two
+    superblocks keep 32 x 64 over 32 x 48."""
+    def kind(m, n, k):
+        return F.qmatmul_plan(dev, O.Q4K, m, n, k, 1 << 20)[1]
+
+    narrow, wide = kind(8, 8192, 256), kind(8, 24592, 2304)
+    assert narrow != wide
+    for m, n, last in [(5, 8193, 2048), (8, 10752, 1792), (12, 12288, 1536), (16, 14336, 1280), (5, 16384, 1280)]:
+        assert kind(m, n, 256) == kind(m, n, 768) == kind(m, n, last) == wide
+        assert kind(m, n, last + 256) == kind(m, n, 7936) == narrow
+    assert kind(3, 16385, 256) == kind(8, 24576, 512) == narrow  # past two a CU: any length
+    for n in (8193, 12288):
+        assert kind(17, n, 256) == kind(32, n, 512) == kind(32, 16384, 4096) != kind(17, n, 768)
 
 
 @pytest.mark.parametrize("m", [64, 128])
