@@ -163,6 +163,13 @@ def device_experts(dev, dt, e, rows, cols, seed, stream):
     (11, 256, 512, 7, 2, O.Q8_0),
     (2, 256, 8192, 4, 2, O.Q4K),          # an entry's blocks past 32 lanes: indexed down + combine kernel
     (1, 512, 256, 300, 16, O.Q4K),        # 16 entries: four passes of the fused down + combine
+    # the grouped path past 128 experts: every width of the routing + quantize launch, and the
+    # batches of more than 256 experts with the tile table
+    (120, 512, 256, 200, 4, O.Q4K),
+    (80, 512, 256, 300, 8, O.Q4K),
+    (61, 256, 512, 400, 7, O.Q6K),
+    (150, 256, 256, 520, 8, O.Q4K),
+    (401, 256, 256, 1000, 5, O.Q4K),
 ])
 def test_moe_ffn(dev, t, d, ffn, e, k, dt):
     say("moe_ffn", t, d, ffn, e, k, dt)

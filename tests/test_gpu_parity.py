@@ -383,6 +383,57 @@ def test_device_quantize_few_blocks(dev, dt, blocks):
         assert np.array_equal(q.dequantize_f16(w.size).numpy(), values.astype(np.float16).view(np.uint16))
 
 
+def extreme_rows(rng):
+    """256-element rows at the ends of the f32 range: Q6_K's search divides by
+    sums near x^3, so 1e-14 and 3e-14 make them denormal and 4e11 and 6e11 put
+    them where a reciprocal is (2^126 .. 2^128); rows of larger and smaller
+    magnitudes, of any bit pattern, and with infinities and NaN."""
+    rows = [rng.standard_normal(256) * s for s in (1e-14, 3e-14, 1e-13, 2e11, 4e11, 6e11, 1e-38, 1e-20, 1e20, 5e37)]
+    for v in (np.inf, -np.inf, np.nan):
+        for n in (1, 3, 40):
+            x = rng.standard_normal(256)
+            x[rng.permutation(256)[:n]] = v
+            rows.append(x)
+    x = rng.standard_normal(256)
+    x[[3, 77, 200]] = [np.inf, -np.inf, np.nan]
+    rows.append(x)
+    rows += [np.full(256, v) for v in (np.inf, -np.inf, np.nan, 3e38, -1e-44)]
+    return np.concatenate([np.stack(rows).astype(np.float32),
+                           rng.integers(0, 1 << 32, (24, 256), dtype=np.uint32).view(np.float32)])
+
+
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+def test_device_quantize_extreme_rows(dev, dt):
+    """from_float, and from_float_imatrix with importance weights of ordinary,
+    huge and denormal size, byte for byte over extreme_rows."""
+    say("device from_float, extreme rows", dt)
+    rng = np.random.default_rng(17)
+    w = extreme_rows(rng)
+    g = w[:6].reshape(-1, 16).astype(np.float64)  # the search's first sum x^3 code, per group
+    big = np.take_along_axis(g, np.abs(g).argmax(1)[:, None], 1)
+    den = np.abs((g ** 3 * np.round(-32 * g / big)).sum(1))
+    assert (den < 2.0 ** -126).sum() > 8 and ((den > 2.0 ** 126) & (den < 3.4e38)).sum() > 8
+    with np.errstate(all="ignore"):
+        want = O.quantize(dt, w)
+    q = dev.qzeros(w.size, dt)
+    q.quantize(dev.from_numpy(w))
+    say("  from_float")
+    assert_blocks(dt, q.data(), want)
+    for size in (1.0, 3e35, 1e-41):
+        qw = (rng.uniform(0.1, 4.0, 256) * size).astype(np.float32)
+        with np.errstate(all="ignore"):
+            want = O.quantize_imatrix(dt, w, qw, 256)
+        q.quantize_imatrix(dev.from_numpy(w), qw, 256)
+        say("  imatrix of size", size)
+        assert_blocks(dt, q.data(), want)
+
+
+def assert_blocks(dt, got, want):
+    got = np.frombuffer(got, O.BLOCK_DTYPE[dt]).reshape(want.shape)
+    bad = np.nonzero(got.view(np.uint8).reshape(got.size, -1) != want.view(np.uint8).reshape(want.size, -1))
+    assert got.tobytes() == want.tobytes(), f"first differing blocks {np.unique(bad[0])[:8]}"
+
+
 def test_device_quantize_known_answers(dev):
     """The hand-derived known-answer blocks of weight_kat.py (grid-exact
     sub-blocks, clamps, ties, saturation, zero blocks) through the device
