@@ -96,7 +96,7 @@ __device__ __forceinline__ int wave_incl_scan(int x, int lane) {
 // a chunk every expert owns a bitmap over the chunk's entries; an entry's rank
 // within its expert is the entries already placed by earlier chunks plus the
 // set bits below it (prefix popcounts), which keeps (token, slot) order.
-__global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __restrict__ ids, int P, int E, int topk,
+__global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __restrict__ ids, unsigned P, int E, int topk,
                                                               int wpe, int* __restrict__ offsets,
                                                               int* __restrict__ sorted_token,
                                                               int* __restrict__ sorted_slot,
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __rest
         fill[e] = 0;
     }
     __syncthreads();
-    for (int i = tid; i < P; i += BATCH_WG) {
+    for (size_t i = tid; i < P; i += BATCH_WG) {
         const int e = ids[i];
         if ((unsigned)e < (unsigned)E) atomicAdd(&off[e], 1);
     }
@@ -150,14 +150,13 @@ __global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __rest
     }
     __syncthreads();
 
-    const int chunk = 32 * wpe;
-    for (int c0 = 0; c0 < P; c0 += chunk) {
-        const int c1 = min(P, c0 + chunk);
+    const unsigned chunk = 32 * wpe;
+    for (unsigned c0 = 0; c0 < P; c0 += chunk) {
+        const unsigned c1 = min(P, c0 + chunk);
         for (int i = tid; i < E * wpe; i += BATCH_WG) bits[i] = 0u;
         __syncthreads();
-        for (int i = c0 + tid; i < c1; i += BATCH_WG) {
-            const int e = ids[i];
-            const int r = i - c0;
+        for (unsigned r = tid; r < c1 - c0; r += BATCH_WG) {
+            const int e = ids[c0 + r];
             if ((unsigned)e < (unsigned)E) atomicOr(&bits[e * wpe + (r >> 5)], 1u << (r & 31));
         }
         __syncthreads();
@@ -170,14 +169,15 @@ __global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __rest
             tot[e] = run;
         }
         __syncthreads();
-        for (int i = c0 + tid; i < c1; i += BATCH_WG) {
+        for (unsigned r = tid; r < c1 - c0; r += BATCH_WG) {
+            const unsigned i = c0 + r;
             const int e = ids[i];
             if ((unsigned)e >= (unsigned)E) continue;
-            const int r = i - c0, wd = e * wpe + (r >> 5);
+            const int wd = e * wpe + (r >> 5);
             const int rank = fill[e] + pc[wd] + __popc(bits[wd] & ((1u << (r & 31)) - 1u));
             const int pos = off[e] + rank;
-            sorted_token[pos] = i / topk;
-            if (sorted_slot) sorted_slot[pos] = i;
+            sorted_token[pos] = (int)(i / (unsigned)topk);
+            if (sorted_slot) sorted_slot[pos] = (int)i;
             entry_expert[pos] = e;
             entry_pos[i] = pos;
         }
@@ -188,20 +188,40 @@ __global__ __launch_bounds__(BATCH_WG) void moe_batches_kernel(const int* __rest
 }
 
 // The same batches for E <= 256 experts: workgroup c places the entries of chunk
-// c (per of them, a multiple of 256; at most 256 chunks) on its own.  It counts all P entries per expert (LDS
-// adds: the totals give every expert's offset and tiles) and those before its
-// chunk; within the chunk, the lanes of a wavefront holding the same expert are
-// found by eight ballots over the id's bits (the lanes that agree on every
-// bit), and the wavefronts' counts are summed in order, so entries keep their
-// (token, slot) order within an expert, as build_expert_batches does.
+// c (a multiple of 256 of them; at most 256 chunks) on its own.  It counts all
+// P entries per expert (LDS adds: the totals give every expert's offset and
+// tiles) and those before its chunk; within the chunk, the lanes of a wavefront
+// holding the same expert are found by eight ballots over the id's bits (the
+// lanes that agree on every bit), and the wavefronts' counts are summed in
+// order, so entries keep their (token, slot) order within an expert, as
+// build_expert_batches does.
 // Workgroup 0 also writes the offsets and the tile table.  One workgroup
 // walking the chunks took 12.5 us for 4096 entries (a chain of barriers on one
 // CU); every workgroup reading all ids again takes 5.9 us.
 constexpr int RANK_WG = 256, RANK_NW = RANK_WG / 64;
 constexpr int RANK_MAX_EXPERTS = 256;
 
-__global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __restrict__ ids, int P, int E, int topk,
-                                                                   int per, int* __restrict__ offsets,
+// Chunks c < rank_chunks(P) of P entries: [rank_begin, rank_end), per = rank_chunk(P).
+// (Unsigned: the last of nearly 2^31 entries would end past an int.)
+constexpr unsigned rank_chunk(unsigned P) { return RANK_WG * ((P + 256u * RANK_WG - 1) / (256u * RANK_WG)); }
+constexpr unsigned rank_chunks(unsigned P) { return P > 0 ? (P + rank_chunk(P) - 1) / rank_chunk(P) : 1; }
+constexpr __host__ __device__ unsigned rank_begin(unsigned c, unsigned per) { return c * per; }
+constexpr __host__ __device__ unsigned rank_end(unsigned c, unsigned per, unsigned P) {
+    return P - c * per < per ? P : (c + 1) * per;
+}
+constexpr bool rank_covers(unsigned P) {  // the chunks are P's entries in order, none empty
+    unsigned at = 0;
+    for (unsigned c = 0; c < rank_chunks(P); c++) {
+        if (rank_begin(c, rank_chunk(P)) != at || rank_end(c, rank_chunk(P), P) <= at) return false;
+        at = rank_end(c, rank_chunk(P), P);
+    }
+    return at == P;
+}
+static_assert(rank_covers(1) && rank_covers(256) && rank_covers(257) && rank_covers(65536) && rank_covers(65537) &&
+              rank_covers(0x7f800000u) && rank_covers(0x7f800001u) && rank_covers(0x7fffffffu));
+
+__global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __restrict__ ids, unsigned P, int E,
+                                                                   int topk, unsigned per, int* __restrict__ offsets,
                                                                    int* __restrict__ sorted_token,
                                                                    int* __restrict__ sorted_slot,
                                                                    int* __restrict__ entry_expert,
@@ -210,18 +230,17 @@ __global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __
     __shared__ int wcnt[RANK_NW][RANK_MAX_EXPERTS];
     __shared__ int wsum[RANK_NW], tsum[RANK_NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c0 = blockIdx.x * per, c1 = min(P, c0 + per);
+    const unsigned c0 = rank_begin(blockIdx.x, per), c1 = rank_end(blockIdx.x, per, P);
     tot[tid] = 0;  // (RANK_MAX_EXPERTS == RANK_WG)
     bef[tid] = 0;
     __syncthreads();
     constexpr int UN = 8;
-    for (int b0 = 0; b0 < P; b0 += UN * RANK_WG) {
+    for (unsigned b0 = 0; b0 < P; b0 += UN * RANK_WG) {
+        const int* from = ids + b0;
+        const unsigned left = P - b0;
         int v[UN];
 #pragma unroll
-        for (int u = 0; u < UN; u++) {
-            const int q = b0 + u * RANK_WG + tid;
-            v[u] = q < P ? ids[q] : -1;
-        }
+        for (int u = 0; u < UN; u++) v[u] = u * RANK_WG + tid < left ? from[u * RANK_WG + tid] : -1;
 #pragma unroll
         for (int u = 0; u < UN; u++)
             if ((unsigned)v[u] < (unsigned)E) {
@@ -258,11 +277,11 @@ __global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __
             if (tid == E - 1) tiles.ntiles[0] = t0 + nt;
         }
     }
-    for (int i0 = c0; i0 < c1; i0 += RANK_WG) {
+    for (unsigned i0 = c0; i0 < c1; i0 += RANK_WG) {
 #pragma unroll
         for (int w = 0; w < RANK_NW; w++) wcnt[w][tid] = 0;
         __syncthreads();
-        const int i = i0 + tid;
+        const unsigned i = i0 + tid;
         const int e = i < c1 ? ids[i] : -1;
         const bool valid = (unsigned)e < (unsigned)E;
         // rank among the wavefront's entries of the same expert
@@ -279,8 +298,8 @@ __global__ __launch_bounds__(RANK_WG) void moe_batches_rank_kernel(const int* __
         if (valid) {
             int pos = bef[e] + rank;
             for (int w = 0; w < wave; w++) pos += wcnt[w][e];
-            sorted_token[pos] = i / topk;
-            if (sorted_slot) sorted_slot[pos] = i;
+            sorted_token[pos] = (int)(i / (unsigned)topk);
+            if (sorted_slot) sorted_slot[pos] = (int)i;
             entry_expert[pos] = e;
             entry_pos[i] = pos;
         }
@@ -633,18 +652,17 @@ hipError_t launch_moe_batches(const int* ids, int P, int E, int topk, int* offse
                               hipStream_t s) {
     if (E <= 0 || E > MOE_MAX_EXPERTS || topk <= 0) return hipErrorInvalidValue;
     if (E <= RANK_MAX_EXPERTS) {
-        const int groups = (P + RANK_WG - 1) / RANK_WG, per = RANK_WG * ((groups + 255) / 256);
-        const int wgs = P > 0 ? (P + per - 1) / per : 1;  // (no entries: the offsets all the same)
-        hipLaunchKernelGGL(moe_batches_rank_kernel, dim3(wgs), dim3(RANK_WG), 0, s, ids, P, E, topk, per, offsets,
-                           sorted_token, sorted_slot, entry_expert, entry_pos, tiles);
+        const unsigned n = P > 0 ? (unsigned)P : 0u;  // (no entries: one workgroup, the offsets all the same)
+        hipLaunchKernelGGL(moe_batches_rank_kernel, dim3(rank_chunks(n)), dim3(RANK_WG), 0, s, ids, n, E, topk,
+                           rank_chunk(n), offsets, sorted_token, sorted_slot, entry_expert, entry_pos, tiles);
         return hipGetLastError();
     }
     // words per expert per chunk: enough for all P entries when they fit
-    const int need = (P + 31) / 32;
+    const int need = P / 32 + (P % 32 != 0);
     int wpe = BATCH_WORDS / E;
     if (need < wpe) wpe = need > 0 ? need : 1;
-    hipLaunchKernelGGL(moe_batches_kernel, dim3(1), dim3(BATCH_WG), 0, s, ids, P, E, topk, wpe, offsets,
-                       sorted_token, sorted_slot, entry_expert, entry_pos, tiles);
+    hipLaunchKernelGGL(moe_batches_kernel, dim3(1), dim3(BATCH_WG), 0, s, ids, (unsigned)P, E, topk, wpe,
+                       offsets, sorted_token, sorted_slot, entry_expert, entry_pos, tiles);
     return hipGetLastError();
 }
 
