@@ -156,7 +156,7 @@ __device__ __forceinline__ int wave_sum_i(int v) {
 //   d     : f32   [rows][K/blk]    (Q8K: the f32 d; Q8_0: f16 d widened)
 //   bsums : int16 [rows][K/256][16] (Q8K only: sums of 16 consecutive quants)
 //   bsh   : f16   [rows][K/256][16] (Q8K only: the same sums as binary16 bits,
-//           exact since |sum| <= 2032; an MFMA operand of the batched kernel)
+//           exact since |sum| <= 16 * 128 = 2048; an MFMA operand of the batched kernel)
 // ---------------------------------------------------------------------------
 struct ActView {
     int8_t* qs;

@@ -23,14 +23,15 @@ __device__ __forceinline__ void store4(void* y, size_t idx, float a, float b, fl
     }
 }
 
-// Eight values: one 16-byte store of f16, two of f32.
+// Eight values: two 8-byte stores of f16, two 16-byte ones of f32.  (The entry
+// points ask for 4-byte aligned f32 outputs and any f16 ones: the stores rely on
+// the unaligned global access that common.hpp states.)
 template <bool F16>
 __device__ __forceinline__ void store8(void* y, size_t idx, const float (&v)[8]) {
     if constexpr (F16) {
         uint32_t h[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) h[i] = half_bits(v[2 * i]) | (half_bits(v[2 * i + 1]) << 16);
-        // (y may be only 8-byte aligned)
         reinterpret_cast<uint2*>(y)[idx / 4] = uint2{h[0], h[1]};
         reinterpret_cast<uint2*>(y)[idx / 4 + 1] = uint2{h[2], h[3]};
     } else {

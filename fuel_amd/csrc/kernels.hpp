@@ -203,7 +203,7 @@ hipError_t launch_block_isums(int dtype, const uint8_t* w, ActView act, int32_t*
 hipError_t launch_dequantize(int dtype, const uint8_t* w, size_t nblocks, float* y16or32,
                              bool to_f16, hipStream_t s);
 
-// weights.hip: from_float on the device (one thread per superblock), and the
+// weights.hip: from_float on the device (one thread per scale group), and the
 // Philox synthetic-input generator.
 hipError_t launch_quantize_weights(int dtype, const float* x, size_t nblocks, uint8_t* out, hipStream_t s);
 // from_float_imatrix (Q4_K, Q6_K): superblock ib uses the importance weights

@@ -18,7 +18,7 @@
 // its 8-term dot products on the VALU.)  f32 step: y += d_x*(d*isum - dmin*msum).
 //
 // Q6_K.  w_e = (q6_e - 32) * sc_g, with sc_g the int8 scale of 16-element
-// group g, lies in [-4096, 4064]: split w = 256*wh + wl with wl in [-128, 127]
+// group g, lies in [-4064, 4096]: split w = 256*wh + wl with wl in [-128, 127]
 // and wh in [-16, 16], both signed bytes, so
 //   isum = 256 * (X . Wh) + (X . Wl)
 // is two exact int8 GEMMs.  The products are formed two per 16-bit lane with
@@ -584,7 +584,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mmq_dma_kernel(const uint8_t* __
 //
 // isum = 8 (X . Ba) + (X . Bb) as in MmqQ4K; msum = sum_j m_j S_j comes from
 // one f16 MFMA per superblock, K = 16 over the activation's 16-element sums
-// b_i (the quantizer's f16 copy: |b_i| <= 2032 is exact) against m_{i/2}
+// b_i (the quantizer's f16 copy: |b_i| <= 2048 is exact) against m_{i/2}
 // (<= 63): every product and partial sum is an integer below 2^24, exact in
 // the f32 accumulator.
 // The f32 step is MmqQ4K's y += d_x * (d * isum - dmin * msum), the same
@@ -1000,7 +1000,8 @@ __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint
         wsrc[j] = (uint32_t)n * row_bytes + 16u * (uint32_t)(q % 9);
     }
     uint32_t xsrc = 0;  // sums or scales
-    if (wave == 2 || wave == 3) xsrc = 32u * (uint32_t)row_of(32 * (wave - 2) + (lane >> 1)) * (uint32_t)KB + 16u * (uint32_t)(lane & 1);
+    if (wave == 2 || wave == 3)
+        xsrc = 32u * (uint32_t)row_of(32 * (wave - 2) + (lane >> 1)) * (uint32_t)KB + 16u * (uint32_t)(lane & 1);
     if (wave == 4) xsrc = 4u * (uint32_t)row_of(lane) * (uint32_t)KB;
     const uint8_t* qbase = reinterpret_cast<const uint8_t*>(act.qs);
     const uint8_t* sbase = reinterpret_cast<const uint8_t*>(act.bsh);

@@ -115,7 +115,7 @@ __device__ __forceinline__ void q8k_store(const Q8KWave& r, const ActView& act, 
     reinterpret_cast<uint32_t*>(act.qs + sb * QK_K)[lane] = r.packed;
     if ((lane & 3) == 0) {
         act.bsums[sb * 16 + (lane >> 2)] = (int16_t)r.bsum;
-        // (|bsum| <= 2032: exact in f16)
+        // (|bsum| <= 16 * 128 = 2^11: exact in f16)
         if (act.bsh) act.bsh[sb * 16 + (lane >> 2)] = __builtin_bit_cast(uint16_t, (_Float16)(float)r.bsum);
     }
     if (lane == 0) act.d[sb] = r.d;

@@ -13,7 +13,7 @@
 // lane's activation row in row tile rt).  Integer sums per superblock / block
 // are exact:
 //   Q4_K  isum = 8*(X.Ba) + X.Bb, msum = X.Bm  (sc = 8a + b; mins broadcast),
-//   Q6_K  isum = 128*(X.Wh) + X.Wl            (w = (q-32)*sc = 128 wh + wl),
+//   Q6_K  isum = 256*(X.Wh) + X.Wl            (w = (q-32)*sc = 256 wh + wl),
 //   Q8_0  isum = X.Q,
 // then one f32 step per superblock (block): y += d_x * (d*isum - dmin*msum).
 #pragma once

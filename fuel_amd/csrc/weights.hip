@@ -624,8 +624,8 @@ hipError_t launch_quantize_weights_imatrix(int dtype, const float* x, size_t nbl
     if (blocks_per_row == 0 || !imatrix) return hipErrorInvalidValue;
     switch (dtype) {
         case GGML_Q4K:
-            hipLaunchKernelGGL(quantize_q4k_imatrix_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(64), 0, s, x, nblocks, out, imatrix,
-                               blocks_per_row);
+            hipLaunchKernelGGL(quantize_q4k_imatrix_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(64), 0, s, x,
+                               nblocks, out, imatrix, blocks_per_row);
             break;
         case GGML_Q6K:
             hipLaunchKernelGGL(quantize_q6k_weights_kernel, dim3((unsigned)((nblocks + 15) / 16)), dim3(256), 0, s, x,

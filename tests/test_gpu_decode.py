@@ -4,7 +4,7 @@ greedy step, the LLaMA-shaped decoder) against the CPU oracle, through the C ABI
 Bit-exact: the rotated, f16-rounded cache rows the attention kernel appends
 (rope_f32 byte_kernels.rs:1885-1964 has no fused multiply-add; neither has the
 kernel), the greedy token (argmax_dim_f32, first index on ties).  f32: the
-fused QMatMuls within 1e-3 of the CPU output norm (the north-star bound);
+fused QMatMuls within 1e-3 of the CPU output norm (the path's bound);
 attention within 1e-5 (f32 only, no quantization).  Decoder logits: within
 1e-2 of their norm.  GPU and CPU agree to ~1e-8 until an f32 ordering
 difference of that size flips one Q8K activation rounding or one f16
@@ -443,7 +443,7 @@ def test_decoder_teacher_forced_logits(dev, small_decoder):
 
 
 def test_decoder_teacher_forced_layers(dev, small_decoder):
-    """Per-layer parity at the north-star bound: after six forced steps, the
+    """Per-layer parity at the path's bound: after six forced steps, the
     seventh position layer by layer with the CPU path teacher-forced on the
     GPU's residual and caches (test_gpu_prefill.teacher_forced_layers)."""
     from test_gpu_prefill import teacher_forced_layers

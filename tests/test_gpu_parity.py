@@ -2,7 +2,7 @@
 
 Bit-exact: activation int8 quants (Q8K / Q8_0 blocks), per-block integer dot
 sums, dequantized values.  f32 outputs: max |y_gpu - y_cpu| <= 1e-3 * ||y_cpu||_2
-against the oracle's restatement of fuel's CPU
+(the path's tolerance), against the oracle's restatement of fuel's CPU
 matmul<T> (AVX2 vec_dot, k_quants.rs:2284-2331) on the same seeded inputs.
 """
 import functools
@@ -665,8 +665,8 @@ def test_qmatmul_mfma_ragged(dev, dt, batch, m, n, k):
 
 def test_qmatmul_q6k_mfma_extreme_scales(dev):
     """Q6_K blocks at the ends of the code and scale ranges (codes 0 and 63,
-    scales -128 and 127) against the exact integer sum: the 7-bit plane split
-    of (q - 32) * sc must carry the full [-4096, 4064] product range."""
+    scales -128 and 127) against the exact integer sum: the byte plane
+    split of (q - 32) * sc must carry the full [-4064, 4096] product range."""
     say("mfma q6k extremes")
     m, n, k = 32, 64, 512
     rng = np.random.default_rng(5)
