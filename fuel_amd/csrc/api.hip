@@ -493,9 +493,10 @@ int route_and_batch(frq_device* dev, const float* logits, size_t t, size_t e, si
 
 // Beyond this many routed entries per expert on average, the expert
 // projections run as grouped int8-MFMA matmuls (one weight pass per expert
-// tile) instead of one mat-vec per routed row (Qwen3-MoE layer, 128 experts:
-// the mat-vec wins at 128 entries, 72 against 81 us; the grouped tiles from
-// 160 entries, 85 against 89 us).
+// tile) instead of one mat-vec per routed row.  128 experts of 2048 / 768: the
+// mat-vec wins at 128 entries, 65 against 67 us, the grouped tiles from 144,
+// 69 against 88.  (Small experts cross later: 16 of 1024 / 512 at 20 entries
+// 13 us on the mat-vec, 22 on the tiles.)
 constexpr double MOE_MMQ_MIN_ROWS_PER_EXPERT = 1.0;
 
 }  // namespace

@@ -950,11 +950,11 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
 // Activation rows are gathered by the DMA's per-lane offsets.  A tile is as
 // tall as an expert's rows usually reach, so an expert's blocks are read and
 // unpacked once, and the wavefronts work only the 16-row parts that hold rows
-// (RL of them, one code path each): the kernel is bound by its VALU work,
-// mostly the unpacking, which does not depend on the rows.  (Q4K 128 experts,
-// 4096 routed rows, 2048 -> 2 x 768 -> 2048: gate|up 111 -> 75 us, down 61 ->
-// 49 us against 32-row tiles of the register-staged kernel, where experts of
-// 33 or more rows take two tiles and each product three MFMAs.)
+// (RL of them, one code path each).  Bound by memory (Q4K 128 experts, 4096
+// routed rows, 2048 -> 2 x 768 -> 2048: gate|up 67.5 us at 4.25 TB/s of counted
+// traffic, down 41.0 at 4.39, a large copy reaching 4.73; 111 and 61 us in
+// 32-row tiles of the register-staged kernel, where experts of 33 or more rows
+// take two tiles and each product three MFMAs).
 constexpr int GRP_RT = 4, GRP_NW = 8;
 
 __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint8_t* __restrict__ W, ActView act,
