@@ -1,4 +1,4 @@
-"""Benchmark of the MI355X quantized mat-vec path.
+"""Benchmark of the MI355X quantized mat-vec path (one row, 7B layer shapes).
 
 A step is one pass of fuel's QMatMul forward at M = 1 (activation quantize to
 Q8K + Q4_K block-dot mat-vec, one fused kernel per matrix) over the four
@@ -14,11 +14,11 @@ kernel (the 4096x32000 Q4_K mat-vec) timed alone the same way.  `cpu_baseline`
 is the oracle's restatement of fuel's CPU path (matmul<BlockQ4K> with the AVX2
 vec_dot) on the host cores, on the same four shapes.
 
-The same shapes are then timed with Q6_K weights (`per_shape_q6k`, the rest
-of config 2), and config 3's M = 32/128/512 rows run on both formats
+The same shapes are then timed with Q6_K weights (`per_shape_q6k`), and
+M = 32/128/512 rows run on both formats
 (`batched.Q4_K`, `batched.Q6_K`: the int8-MFMA path).
 
-The same run measures BASELINE config 4 (`decode`): greedy decode of a
+The same run measures decoding (`decode`): greedy decode of a
 random-init LLaMA-2-7B-shaped Q4_K_M-mix decoder after a 512-token prompt,
 256 generated tokens timed, with fuel's CPU path (the oracle's restatement)
 timed on the same weights and KV state beside it (`decode.cpu_baseline`).
@@ -196,7 +196,7 @@ def gpu_leg(steps: int, warmup: int, q6k: bool = True):
         batched["Q4_K"] = batched_leg(hip, dev, stream, mats)
     mats.clear()  # frees the rotated weights
     per_shape_q6k = None
-    if q6k:  # config 2's Q6_K sweep and config 3's Q6_K rows
+    if q6k:  # the Q6_K sweep and its M = 32/128/512 rows
         mats = make_mats(dev, F.Q6K, 700)
         per_shape_q6k = shape_times(hip, dev, stream, mats)
         say(f"[bench] Q6_K sweep {per_shape_q6k}")
@@ -212,7 +212,7 @@ INT8_PEAK_TOPS = 5000.0
 
 
 def batched_leg(hip, dev, stream, mats):
-    """BASELINE config 3: QMatMul with M = 32, 128, 512 activation rows at the
+    """QMatMul with M = 32, 128, 512 activation rows at the
     same shapes and rotated weights (the int8-MFMA path), and small batches
     M = 2, 4, 8, 16 (the one-pass small-batch mat-vec below 16 rows).
     Reported as useful TOPS (2 M N K per call) against the dense int8 peak and
@@ -262,7 +262,7 @@ MOE_T = (1, 16, 512)
 
 
 def moe_leg():
-    """BASELINE config 5: Qwen3-MoE-style expert layer, 128 experts, top-8 of
+    """Qwen3-MoE-style expert layer, 128 experts, top-8 of
     N(0,1) router logits, d 2048, expert FFN 768, Q4_K experts from N(0,0.02);
     T = 1, 16, 512 tokens.  Four copies of the 340 MB expert set are rotated
     (1.36 GB, beyond the Infinity Cache) and every call routes fresh logits.
@@ -445,7 +445,7 @@ DECODE_NEW = 256
 
 
 def decode_leg(new_tokens: int = DECODE_NEW, prompt_len: int = DECODE_PROMPT):
-    """random-init LLaMA-2-7B-shaped decoder (Q4_K_M-style
+    """Random-init LLaMA-2-7B-shaped decoder (Q4_K_M-style
     mix), a 512-token uniform random prompt, greedy decode of `new_tokens`.
     Every step is one replay of a captured HIP graph (162 launches); the
     prompt is run through the same step with its tokens forced.  Timed: the
@@ -546,7 +546,7 @@ def counter_refs() -> dict:
 
 
 def decode_breakdown_leg(new_tokens: int = 128, prompt_len: int = DECODE_PROMPT) -> dict:
-    """Per-kernel-class time of the config-4 decode step, from HIP events in
+    """Per-kernel-class time of the 7B decode step, from HIP events in
     the process: the decoder is run to position prompt_len + new_tokens (the
     prompt forced, then greedy steps), then each class of the step's launches
     (LlamaDecoder.STEP_PARTS: the q|k + v pair, attention with the
@@ -719,7 +719,7 @@ def cpu_leg(target_s: float):
 
 
 def cpu_config1_leg(target_s: float):
-    """BASELINE config 1 on fuel's CPU path itself: matmul<BlockQ8_0> (the
+    """The Q8_0 4096 x 4096 QMatMul on fuel's CPU path itself: matmul<BlockQ8_0> (the
     oracle restatement with the AVX2 vec_dot_q8_0_q8_0, avx.rs:72-88) of
     x [1, 4096] ~ N(0, 1) against W [4096, 4096] ~ N(0, 0.02) quantized by
     BlockQ8_0::from_float, on the host cores; median of repeated calls, the
@@ -772,12 +772,12 @@ def main() -> int:
     ap.add_argument("--copy-bytes", type=int, default=0,
                     help="first run device copies of this size (counter calibration)")
     ap.add_argument("--no-decode", action="store_true")
-    ap.add_argument("--no-batched", action="store_true", help="skip the config-3 M = 32/128/512 leg")
-    ap.add_argument("--no-moe", action="store_true", help="skip the config-5 MoE leg")
+    ap.add_argument("--no-batched", action="store_true", help="skip the M = 32/128/512 leg")
+    ap.add_argument("--no-moe", action="store_true", help="skip the MoE leg")
     ap.add_argument("--no-q6k", action="store_true", help="skip the Q6_K sweep and Q6_K batched rows")
-    ap.add_argument("--decode-only", action="store_true", help="run only the config-4 decode legs")
+    ap.add_argument("--decode-only", action="store_true", help="run only the 7B decode legs")
     ap.add_argument("--decode-breakdown", action="store_true",
-                    help="time each kernel class of the config-4 decode step (HIP events) and print its JSON line")
+                    help="time each kernel class of the 7B decode step (HIP events) and print its JSON line")
     ap.add_argument("--probe", default=None, metavar="K,N,DTYPE,M",
                     help="time one QMatMul configuration alone (profiling runs) and print its JSON line")
     ap.add_argument("--probe-read", default=None, metavar="BYTES[,WG_PER_CU,UNROLL[,NT]]",
@@ -813,7 +813,7 @@ def main() -> int:
         say(f"[bench] decode {dres}")
         if not args.no_cpu:
             dres["cpu_baseline"] = cpu_decode_leg(dec, tokens, logits0, args.cpu_seconds)
-        print(json.dumps({"metric": "decode tokens/s, LLaMA-2-7B-shaped Q4_K_M mix (BASELINE config 4)",
+        print(json.dumps({"metric": "decode tokens/s, LLaMA-2-7B-shaped Q4_K_M mix",
                           "value": dres["tokens_per_s"], "unit": "tokens/s", "decode": dres}), flush=True)
         return 0
     global BATCHED_M
@@ -845,7 +845,7 @@ def main() -> int:
         "data": "synthetic: Philox-4x32-10 N(0,1) activations, N(0,0.02) weights quantized to Q4_K on the device "
                 "by the from_float port (bit-exact with the CPU quantizer)",
         "config": {
-            "workload": "Q4_K batch-1 QMatMul sweep at LLaMA-2-7B layer shapes (BASELINE config 2)",
+            "workload": "Q4_K batch-1 QMatMul sweep at LLaMA-2-7B layer shapes",
             "shapes_KxN": [f"{k}x{n}" for k, n in SHAPES],
             "m": 1,
             "weight_rotation_copies": rot,
@@ -875,7 +875,7 @@ def main() -> int:
         say(f"[bench] read ceiling {rc}")
     if batched:
         out["batched"] = batched
-    if not args.shape:  # BASELINE config 1's QMatMul (Q8_0 [1,4096] x [4096,4096]) on the device
+    if not args.shape:  # the Q8_0 [1,4096] x [4096,4096] QMatMul on the device
         c1 = probe_leg(4096, 4096, 8, 1)
         c1_bytes = algo_bytes(4096, 4096, 34, 32)
         out["config1_q8_0_4096x4096"] = {"us": c1["us"], "GB_s": round(c1_bytes / c1["us"] / 1e3, 1),
@@ -884,7 +884,7 @@ def main() -> int:
             c1cpu = cpu_config1_leg(min(3.0, args.cpu_seconds))
             out["config1_q8_0_4096x4096"]["cpu_baseline"] = c1cpu
             out["config1_q8_0_4096x4096"]["gpu_over_cpu"] = round(c1cpu["us"] / c1["us"], 1)
-        say(f"[bench] config 1 {out['config1_q8_0_4096x4096']}")
+        say(f"[bench] Q8_0 4096x4096 {out['config1_q8_0_4096x4096']}")
     if not args.no_moe:
         out["moe"] = moe_leg()
         say(f"[bench] moe {out['moe']}")

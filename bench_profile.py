@@ -1,4 +1,4 @@
-"""Profiling runs behind bench.py's roofline figures (run on the GPU box).
+"""Profiling runs behind bench.py's roofline figures (run where the GPU is).
 
 Three rocprofv3 passes over bench.py restricted to one shape:
   1. --kernel-trace --stats      -> average duration of the mat-vec kernel;
@@ -9,8 +9,8 @@ the factor that converts FETCH_SIZE / WRITE_SIZE to bytes.  Writes a Markdown
 summary and a JSON file (traffic bytes per launch) into --out.
 
 With --leg decode / batched / moe it instead runs one --kernel-trace --stats
-pass over that bench.py leg (config 4 decode + batched prompt, config 3
-M = 32/128/512 matmuls, config 5 MoE layer) and writes the per-kernel summary.
+pass over that bench.py leg (7B decode + batched prompt, M = 32/128/512
+matmuls, MoE layer) and writes the per-kernel summary.
 
 With --leg counters it runs a kernel trace and counter passes (instruction
 mix, MFMA busy and int8 MOPS, LDS conflicts, waits, HBM bytes) over one QMatMul
@@ -53,12 +53,12 @@ def rows(d: str, name: str):
 # one kernel-trace pass per leg: (bench.py arguments, summary file name, title)
 LEGS = {
     "decode": (["--decode-only", "--no-cpu"], "decode_7b_q4km",
-               "Config 4: 7B Q4_K_M decode (512-token batched prompt, 512 forced steps, 256 greedy tokens)"),
+               "7B Q4_K_M decode (512-token batched prompt, 512 forced steps, 256 greedy tokens)"),
     "batched": (["--shape", "4096x4096", "--steps", "5", "--warmup", "1", "--no-cpu", "--no-decode", "--no-moe"],
                 "mmq_batched_m32_m128_m512",
-                "Config 3: Q4_K / Q6_K QMatMul at M = 32, 128, 512 (int8 MFMA), 7B layer shapes"),
+                "Q4_K / Q6_K QMatMul at M = 32, 128, 512 (int8 MFMA), 4096 x 4096"),
     "moe": (["--shape", "4096x4096", "--steps", "5", "--warmup", "1", "--no-cpu", "--no-decode", "--no-batched",
-             "--no-q6k"], "moe_qwen3_layer", "Config 5: Qwen3-MoE layer (route, gate|up, down, combine) at T = 1/16/512"),
+             "--no-q6k"], "moe_qwen3_layer", "Qwen3-MoE layer (route, gate|up, down, combine) at T = 1/16/512"),
 }
 
 
@@ -193,7 +193,7 @@ def counters_leg(probe: str, pattern: str, out: str, summarize_only: bool) -> in
 
 
 def breakdown_leg(out: str, summarize_only: bool) -> int:
-    """Config-4 decode step per kernel class from HIP events in the process
+    """7B decode step per kernel class from HIP events in the process
     (bench.py --decode-breakdown), without a profiler."""
     name = "decode_7b_q4km_breakdown"
     cmd = ["python3", "bench.py", "--decode-breakdown"]
@@ -207,7 +207,7 @@ def breakdown_leg(out: str, summarize_only: bool) -> int:
     if res is None:
         raise SystemExit(f"no JSON line in {log}")
     with open(os.path.join(ROOT, out, f"{name}.md"), "w") as f:
-        f.write("# Config 4: decode step of the 7B-shaped Q4_K_M decoder, per kernel class\n\n")
+        f.write("# Decode step of the 7B-shaped Q4_K_M decoder, per kernel class\n\n")
         f.write(f"Made by `python3 bench_profile.py --leg decode_breakdown` (repository root, one MI355X), which runs "
                 f"`{' '.join(cmd)}`: HIP events around graph replays of each class of the step's launches over all "
                 f"32 layers (a class of one launch per token captured 16 times per graph, so that the host's "

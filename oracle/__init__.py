@@ -1,6 +1,6 @@
 """ctypes front-end of the CPU oracle (oracle/fuel_oracle.c).
 
-TEST INFRASTRUCTURE ONLY: the checker for the HIP path and the source of the
+TEST INFRASTRUCTURE ONLY: the oracle of the HIP path and the source of the
 CPU baseline.  Only tests/, ``__graft_entry__.smoke()`` and bench.py's
 ``cpu_baseline`` leg import this package.  The product (fuel_amd/) never does.
 

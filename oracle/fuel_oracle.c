@@ -1,7 +1,7 @@
 /*
  * fuel_oracle.c -- CPU restatement of fuel's quantized-matmul path.
  *
- * TEST INFRASTRUCTURE ONLY (the checker and the CPU baseline).  The product
+ * TEST INFRASTRUCTURE ONLY (the oracle and the CPU baseline).  The product
  * library under fuel_amd/ never includes, links or calls this file.
  *
  * Build: see oracle/Makefile.  It MUST be compiled with -ffp-contract=off and

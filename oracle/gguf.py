@@ -1,4 +1,4 @@
-"""GGUF reader and writer in plain Python: test infrastructure (the checker of
+"""GGUF reader and writer in plain Python: test infrastructure (the oracle of
 the library's native reader and the maker of test files), never product code.
 
 `read` restates fuel_formats::gguf::Content::read (fuel-formats/src/

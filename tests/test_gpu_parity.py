@@ -174,7 +174,7 @@ def test_qmatmul_q8_0_batched(dev, m):
 
 
 def test_qmatmul_q8_0_config1(dev):
-    # BASELINE config 1: Q8_0 QMatMul, x [1,4096] ~ N(0,1), W [4096,4096] ~ N(0,0.02)
+    # Q8_0 QMatMul, x [1,4096] ~ N(0,1), W [4096,4096] ~ N(0,0.02)
     k = n = 4096
     wq = weights(O.Q8_0, n, k)
     x = acts(1, k)
@@ -485,7 +485,7 @@ def test_qmatmul_mfma_rows(dev, dt, m):
 @pytest.mark.parametrize("k,n", SHAPES_7B)
 @pytest.mark.parametrize("m", [16, 24, 32, 48, 96, 128, 160, 200, 512])
 def test_qmatmul_mfma_7b_shapes(dev, dt, k, n, m):
-    """BASELINE config 3: M = 32 / 128 / 512 rows at the four 7B shapes (the
+    """M = 32 / 128 / 512 rows at the four 7B shapes (the
     43-superblock rows of K = 11008, split K, the LDS-DMA staging), 16 / 24
     rows (the tiled kernel's partly empty 32-row tiles for the wide matrices,
     the skinny kernel at N = 4096), and 48 / 96 / 160 / 200 rows: Q4_K's 32 x

@@ -171,7 +171,7 @@ def test_decoder_prefill_matches_steps(dev, prefill_pair, plen):
         assert rel_err(pre.logits.numpy(), step.logits.numpy()) < DEC_TOL
 
 
-# ---- the full config-4 model ----
+# ---- the full 7B-shaped model ----
 
 # The 7B-shaped decoder after 32 layers: the GPU and CPU paths compute every
 # matmul from the same blocks with exact integer sums, but in different f32
@@ -185,7 +185,7 @@ FULL_TOL = 6e-3
 
 
 def test_full_7b_decoder_prefill_and_steps(dev):
-    """BASELINE config 4 at full size (32 layers, d 4096, 32 heads, FFN 11008,
+    """The 7B-shaped decoder at full size (32 layers, d 4096, 32 heads, FFN 11008,
     vocab 32000, Q4_K_M mix): a 512-token uniform random prompt through the
     batched prefill (int8-MFMA projections, 512-row attention), then two
     greedy steps from the captured-graph decode path's state, against the
