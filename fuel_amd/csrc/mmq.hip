@@ -657,60 +657,38 @@ __device__ __forceinline__ int bytes_times_p(uint32_t q, uint32_t f2) {
 }
 
 // What both wide-tile kernels do with a weight column of a superblock, so that
-// they give the same bits.  Lane group kb (16 lanes) of column `col`:
-struct WideHead {  // d, dmin, the 6-bit scales split as 8 a + b, the lane group's mins
-    float d, dmin;
-    uint32_t aw[2], bw[2], mw;
-};
-__device__ __forceinline__ WideHead wide_head(const uint8_t* col, int kb) {
+// they give the same bits.  (Plain references and scalars: gathered in structs
+// they changed the compiler's schedule, 8 rows of 4096 x 11008 +0.5%.)
+// d, dmin, the 6-bit scales split as 8 a + b, lane group kb's mins:
+__device__ __forceinline__ void wide_head(const uint8_t* col, int kb, float& d, float& dmin, uint32_t (&aw)[2],
+                                          uint32_t (&bw)[2], uint32_t& mw) {
     const uint4 hd = *reinterpret_cast<const uint4*>(col);
     const uint32_t sc0 = hd.y & 0x3f3f3f3fu;
     const uint32_t sc1 = (hd.w & 0x0f0f0f0fu) | (((hd.y >> 6) & 0x03030303u) << 4);
     const uint32_t mn0 = hd.z & 0x3f3f3f3fu;
     const uint32_t mn1 = ((hd.w >> 4) & 0x0f0f0f0fu) | (((hd.z >> 6) & 0x03030303u) << 4);
-    WideHead h;
-    h.d = f16_to_f32(hd.x & 0xffffu);
-    h.dmin = f16_to_f32(hd.x >> 16);
-    h.aw[0] = (sc0 >> 3) & 0x07070707u;
-    h.aw[1] = (sc1 >> 3) & 0x07070707u;
-    h.bw[0] = sc0 & 0x07070707u;
-    h.bw[1] = sc1 & 0x07070707u;
-    h.mw = kb < 2 ? mn0 : mn1;
-    return h;
+    d = f16_to_f32(hd.x & 0xffffu);
+    dmin = f16_to_f32(hd.x >> 16);
+    aw[0] = (sc0 >> 3) & 0x07070707u;
+    aw[1] = (sc1 >> 3) & 0x07070707u;
+    bw[0] = sc0 & 0x07070707u;
+    bw[1] = sc1 & 0x07070707u;
+    mw = kb < 2 ? mn0 : mn1;
 }
-struct WideSel {
-    uint32_t s0, s1;  // v_perm selectors of scale byte 2 (kb>>1) + (t>>1), K steps t < 2 and t >= 2
-    uint32_t m;       // msum B operand: bytes 2 (kb&1), 2 (kb&1) + 1 of min word kb>>1
-};
-__device__ __forceinline__ WideSel wide_sel(int kb) {
-    const uint32_t s0 = (uint32_t)(2 * (kb >> 1)) * 0x00010001u | 0x0c000c00u;
-    return {s0, s0 + 0x00010001u, (uint32_t)(2 * (kb & 1)) * 0x01010101u + 0x01010000u};
+// the B operand of 16 codes times a factor
+__device__ __forceinline__ v4i wide_plane(const uint32_t (&qd)[4], uint32_t p) {
+    return v4i{bytes_times_p(qd[0], p), bytes_times_p(qd[1], p), bytes_times_p(qd[2], p), bytes_times_p(qd[3], p)};
 }
-// the B operands of K step t: the codes times a and times b
-__device__ __forceinline__ void wide_planes(const uint8_t* col, const WideHead& h, const WideSel& s, int kb, int t,
-                                            v4i& ba, v4i& bb) {
-    const uint4 rw = *reinterpret_cast<const uint4*>(col + 16 + 64 * (t & 1) + 16 * kb);
-    const uint32_t sh = t >= 2 ? 4u : 0u;
-    const uint32_t qd[4] = {(rw.x >> sh) & 0x0f0f0f0fu, (rw.y >> sh) & 0x0f0f0f0fu, (rw.z >> sh) & 0x0f0f0f0fu,
-                            (rw.w >> sh) & 0x0f0f0f0fu};
-    const uint32_t sel = t >= 2 ? s.s1 : s.s0;
-    const uint32_t pa = byte_pair(h.aw[t & 1], sel), pb = byte_pair(h.bw[t & 1], sel);
-    ba = v4i{bytes_times_p(qd[0], pa), bytes_times_p(qd[1], pa), bytes_times_p(qd[2], pa), bytes_times_p(qd[3], pa)};
-    bb = v4i{bytes_times_p(qd[0], pb), bytes_times_p(qd[1], pb), bytes_times_p(qd[2], pb), bytes_times_p(qd[3], pb)};
-}
-__device__ __forceinline__ wh4 wide_mins(const WideHead& h, const WideSel& s) {
-    const uint32_t mm = __builtin_amdgcn_perm(0u, h.mw, s.m);  // bytes m_lo, m_lo, m_hi, m_hi
+// the msum B operand
+__device__ __forceinline__ wh4 wide_mins(uint32_t mw, uint32_t msel) {
+    const uint32_t mm = __builtin_amdgcn_perm(0u, mw, msel);  // bytes m_lo, m_lo, m_hi, m_hi
     return wh4{(_Float16)(mm & 0xffu), (_Float16)((mm >> 8) & 0xffu), (_Float16)((mm >> 16) & 0xffu),
                (_Float16)(mm >> 24)};
 }
-// a 16 x 16 tile's msum, and the f32 step of one of its outputs (as a function
-// over the tile's four outputs the 16-row tiles measured 1% slower)
-__device__ __forceinline__ wf4 wide_msum(const wh4 sa, const wh4 mb) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(sa, mb, wf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-}
-__device__ __forceinline__ float wide_step(float y, float dx, const WideHead& h, float ms, int sa, int sb) {
+// the f32 step of one output, sa and sb its two planes' sums
+__device__ __forceinline__ float wide_step(float y, float dx, float d, float dmin, float ms, int sa, int sb) {
     const int isum = 8 * sa + sb;
-    return fmaf(dx, fmaf(-h.dmin, ms, h.d * (float)isum), y);
+    return fmaf(dx, fmaf(-dmin, ms, d * (float)isum), y);
 }
 
 // KG > 1: KG groups of NW wavefronts share the tile, group g taking every
@@ -818,7 +796,11 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
             }
         });
     };
-    const WideSel sel = wide_sel(kb);
+    // v_perm selectors of scale byte 2 (kb>>1) + (t>>1)
+    const uint32_t sel0 = (uint32_t)(2 * (kb >> 1)) * 0x00010001u | 0x0c000c00u;
+    const uint32_t sel1 = sel0 + 0x00010001u;
+    // msum B operand: bytes 2 (kb&1), 2 (kb&1) + 1 of min word kb>>1
+    const uint32_t msel = (uint32_t)(2 * (kb & 1)) * 0x01010101u + 0x01010000u;
 
     float facc[RT][CT][4];
 #pragma unroll
@@ -850,12 +832,14 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
         // multiplied
         if (b + KG < b1) issue(b + KG, KR == 0 ? slot1 : slot0);
         if (KG > 1 && b >= b1) return;  // (this group has no superblock left)
-        WideHead h[CT];
+        // column headers: d, dmin, the 6-bit scales split as 8 a + b, the mins
+        float d[CT], dmin[CT];
+        uint32_t aw[CT][2], bw[CT][2], mw[CT];
         const uint8_t* col[CT];
 #pragma unroll
         for (int c = 0; c < CT; c++) {
             col[c] = Wl + (16 * (CT * wave + c) + l16) * Q4K_BYTES;
-            h[c] = wide_head(col[c], kb);
+            wide_head(col[c], kb, d[c], dmin[c], aw[c], bw[c], mw[c]);
         }
         v4i acc[RT][CT][2];
 #pragma unroll
@@ -866,8 +850,13 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
             for (int r = 0; r < RT; r++) afr[r] = *reinterpret_cast<const v4i*>(A + (16 * r + l16) * QK_K + 16 * (j ^ l16));
 #pragma unroll
             for (int c = 0; c < CT; c++) {
-                v4i ba, bb;
-                wide_planes(col[c], h[c], sel, kb, t, ba, bb);
+                const uint4 rw = *reinterpret_cast<const uint4*>(col[c] + 16 + 64 * (t & 1) + 16 * kb);
+                const uint32_t sh = t >= 2 ? 4u : 0u;
+                const uint32_t qd[4] = {(rw.x >> sh) & 0x0f0f0f0fu, (rw.y >> sh) & 0x0f0f0f0fu,
+                                        (rw.z >> sh) & 0x0f0f0f0fu, (rw.w >> sh) & 0x0f0f0f0fu};
+                const uint32_t sel = t >= 2 ? sel1 : sel0;
+                const uint32_t pa = byte_pair(aw[c][t & 1], sel), pb = byte_pair(bw[c][t & 1], sel);
+                const v4i ba = wide_plane(qd, pa), bb = wide_plane(qd, pb);
                 const v4i zero = v4i{0, 0, 0, 0};
 #pragma unroll
                 for (int r = 0; r < RT; r++) {
@@ -876,9 +865,12 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
                 }
             }
         }
+        // msum on f16 MFMA, then the f32 step
         wh4 mb[CT];
 #pragma unroll
-        for (int c = 0; c < CT; c++) mb[c] = wide_mins(h[c], sel);
+        for (int c = 0; c < CT; c++) {
+            mb[c] = wide_mins(mw[c], msel);
+        }
 #pragma unroll
         for (int r = 0; r < RT; r++) {
             const wh4 sa = *reinterpret_cast<const wh4*>(S + (16 * r + l16) * 32 + 8 * kb);  // b_{4kb..4kb+3}
@@ -886,10 +878,11 @@ __global__ __launch_bounds__(64 * NW * KG) void mmq_q4k_wide_kernel(const uint8_
             const float dxv[4] = {dx.x, dx.y, dx.z, dx.w};
 #pragma unroll
             for (int c = 0; c < CT; c++) {
-                const wf4 ms = wide_msum(sa, mb[c]);
+                const wf4 ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, mb[c], wf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    facc[r][c][i] = wide_step(facc[r][c][i], dxv[i], h[c], ms[i], acc[r][c][0][i], acc[r][c][1][i]);
+                    facc[r][c][i] = wide_step(facc[r][c][i], dxv[i], d[c], dmin[c], ms[i], acc[r][c][0][i],
+                                              acc[r][c][1][i]);
             }
         }
     };
@@ -1011,7 +1004,9 @@ __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint
     const uint8_t* sbase = reinterpret_cast<const uint8_t*>(act.bsh);
     const uint8_t* dbase = reinterpret_cast<const uint8_t*>(act.d);
 
-    const WideSel sel = wide_sel(kb);
+    const uint32_t sel0 = (uint32_t)(2 * (kb >> 1)) * 0x00010001u | 0x0c000c00u;
+    const uint32_t sel1 = sel0 + 0x00010001u;
+    const uint32_t msel = (uint32_t)(2 * (kb & 1)) * 0x01010101u + 0x01010000u;
     const uint32_t slot0 = lds_addr(sB0), slot1 = lds_addr(sB1);
 
     auto run = [&](auto rl) __attribute__((always_inline)) {
@@ -1044,7 +1039,9 @@ __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint
             compiler_fence();
             if (b + 1 < KB) issue(b + 1, KR == 0 ? slot1 : slot0);
             const uint8_t* col = A + T::OW + (16 * wave + l16) * Q4K_BYTES;
-            const WideHead h = wide_head(col, kb);
+            float d, dmin;
+            uint32_t aw[2], bw[2], mw;
+            wide_head(col, kb, d, dmin, aw, bw, mw);
             v4i acc[RL][2];
 #pragma unroll
             for (int t = 0; t < 4; t++) {
@@ -1053,8 +1050,13 @@ __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint
 #pragma unroll
                 for (int r = 0; r < RL; r++)
                     afr[r] = *reinterpret_cast<const v4i*>(A + (16 * r + l16) * QK_K + 16 * (j ^ l16));
-                v4i ba, bb;
-                wide_planes(col, h, sel, kb, t, ba, bb);
+                const uint4 rw = *reinterpret_cast<const uint4*>(col + 16 + 64 * (t & 1) + 16 * kb);
+                const uint32_t sh = t >= 2 ? 4u : 0u;
+                const uint32_t qd[4] = {(rw.x >> sh) & 0x0f0f0f0fu, (rw.y >> sh) & 0x0f0f0f0fu,
+                                        (rw.z >> sh) & 0x0f0f0f0fu, (rw.w >> sh) & 0x0f0f0f0fu};
+                const uint32_t sel = t >= 2 ? sel1 : sel0;
+                const uint32_t pa = byte_pair(aw[t & 1], sel), pb = byte_pair(bw[t & 1], sel);
+                const v4i ba = wide_plane(qd, pa), bb = wide_plane(qd, pb);
                 const v4i zero = v4i{0, 0, 0, 0};
 #pragma unroll
                 for (int r = 0; r < RL; r++) {
@@ -1062,16 +1064,16 @@ __global__ __launch_bounds__(64 * GRP_NW) void mmq_q4k_grouped_kernel(const uint
                     acc[r][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(afr[r], bb, t == 0 ? zero : acc[r][1], 0, 0, 0);
                 }
             }
-            const wh4 mb = wide_mins(h, sel);
+            const wh4 mb = wide_mins(mw, msel);
 #pragma unroll
             for (int r = 0; r < RL; r++) {
                 const wh4 sa = *reinterpret_cast<const wh4*>(S + (16 * r + l16) * 32 + 8 * kb);  // b_{4kb..4kb+3}
                 const float4 dx = *reinterpret_cast<const float4*>(D + 16 * r + 4 * kb);
                 const float dxv[4] = {dx.x, dx.y, dx.z, dx.w};
-                const wf4 ms = wide_msum(sa, mb);
+                const wf4 ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, mb, wf4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    facc[r][i] = wide_step(facc[r][i], dxv[i], h, ms[i], acc[r][0][i], acc[r][1][i]);
+                    facc[r][i] = wide_step(facc[r][i], dxv[i], d, dmin, ms[i], acc[r][0][i], acc[r][1][i]);
             }
         };
         for (int b = 0; b < KB; b += 2) {
